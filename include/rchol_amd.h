@@ -69,6 +69,11 @@ typedef struct rchol_amd_ctx rchol_amd_ctx;
                                          the default (2^26, ~0.67 s).  A lower bound turns
                                          longer waits into RCHOL_AMD_ESTALL: for testing
                                          the error path */
+#define RCHOL_AMD_OPT_MERGE 12        /* 1 (default): the next upload_G merges consecutive narrow
+                                         levels of the single-right-hand-side sweeps into
+                                         groups of one handshake each, where the factor's
+                                         signs allow it; 0: it does not (a shorter upload, for
+                                         a factor that is used once) */
 
 /* Counters filled by rchol_amd_get_stats. */
 typedef struct rchol_amd_stats {
@@ -277,6 +282,17 @@ void rchol_amd_schedule_free(rchol_amd_schedule *s);
 int rchol_amd_chunk_apply_host(size_t n, const size_t *colPtr, const size_t *rowIdx,
                                const double *val, int max_rows, const double *r, double *z,
                                int *counts, long long *rounds, double *est_us);
+
+/* Host-only: the merged-level plan of the persistent sweeps for a stored
+ * factor (consecutive narrow levels merged into groups whose rows read only
+ * earlier groups), executed on the CPU: z = G^-T G^-1 r.  A row that reads
+ * its own or a later group is RCHOL_AMD_EINVAL.  groups[2] (levels, where
+ * nothing is merged), entries[2] (of merged rows) and est_us[2] (estimates in
+ * microseconds) of the forward and the backward sweep may be NULL.  For
+ * tests; no reference counterpart. */
+int rchol_amd_merge_apply_host(size_t n, const size_t *colPtr, const size_t *rowIdx,
+                               const double *val, const double *r, double *z, int *groups,
+                               long long *entries, double *est_us);
 
 /* Number of visible HIP devices (0 when none); never fails. */
 int rchol_amd_device_count(void);

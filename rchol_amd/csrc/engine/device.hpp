@@ -105,163 +105,216 @@ __device__ long long g_wait_ticks = kWaitTicks;
 constexpr int kPollCap = RCHOL_AMD_POLL_CAP;
 
 
+// The bound and back-off of one wait.
+struct Poll {
+  long long t0 = 0;
+  int polls = 0, backoff = 1;
+  // after a failed poll: every 8th time, whether the wait must end (past its
+  // bound, or the error flag is up)
+  __device__ __forceinline__ bool expired(const int *err) {
+    if (polls == 0) t0 = wall_clock64();
+    return (++polls & 7) == 0 &&
+           (wall_clock64() - t0 > g_wait_ticks ||
+            __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  }
+  // doubling back-off up to cap units of 64 clocks
+  __device__ __forceinline__ void sleep(int cap) {
+    for (int i = 0; i < backoff; i++) __builtin_amdgcn_s_sleep(1);
+    if (backoff < cap) backoff <<= 1;
+  }
+};
+
+// Waits until *p is published (the same p in every active lane: one request
+// per poll), with back-off and a bound that raises the error flag.
+template <typename T>
+__device__ __forceinline__ void await_value(const T *p, int *err) {
+  Poll w;
+  while (Sent<T>::is(Sent<T>::load_agent(p))) {
+    if (w.expired(err)) {
+      atomicOr(err, 1);
+      break;
+    }
+    w.sleep(kPollCap);
+  }
+}
+
+// Re-reads the pending slots of a round (j[u] < 0: an unused slot) and
+// returns the lanes that still hold a sentinel.
+template <typename T, int U>
+__device__ __forceinline__ unsigned long long pending_lanes(const int (&j)[U], const T (&xv)[U]) {
+  bool pend = false;
+#pragma unroll
+  for (int u = 0; u < U; u++) pend |= j[u] >= 0 && Sent<T>::is(xv[u]);
+  return __ballot(pend);
+}
+template <typename T, int U>
+__device__ __forceinline__ unsigned long long reread_pending(const T *x, const int (&j)[U],
+                                                             T (&xv)[U], int stride = 1) {
+#pragma unroll
+  for (int u = 0; u < U; u++)
+    if (j[u] >= 0 && Sent<T>::is(xv[u])) xv[u] = Sent<T>::load_agent(x + (size_t)j[u] * stride);
+  return pending_lanes(j, xv);
+}
+template <typename T, int U>
+__device__ __forceinline__ void zero_pending(const int (&j)[U], T (&xv)[U]) {
+#pragma unroll
+  for (int u = 0; u < U; u++)
+    if (j[u] >= 0 && Sent<T>::is(xv[u])) xv[u] = T(0);
+}
+
 // Completes a round of U gathers per lane, xv[u] = x[j[u]] (j[u] < 0: an
 // unused slot), once some lane of the wave still holds a sentinel.  Called
-// by the whole wave, converged.  Pending slots are re-read coherently first
-// (a plain load may have hit a line cached before publication); while some
-// remain, one lane polls the first pending address of the wave with
-// back-off, and once that value is there every lane re-reads all of its
-// pending slots at once (one load latency for the whole round).  A wait
-// longer than g_wait_ticks raises the error flag; a raised flag zeroes what is
-// still pending and returns.
+// by the whole wave, converged.  One lane polls the first pending address of
+// the wave (a plain load may have hit a line cached before publication: then
+// the first poll succeeds), and once that value is there every lane re-reads
+// all of its pending slots at once, one load latency for the whole round.
+// The slots are not re-read before that poll: most waits are long, and the
+// re-reads of waves that are early load the fabric that the publications
+// travel on.  A wait longer than g_wait_ticks raises the error flag; a raised
+// flag zeroes what is still pending and returns.
 // Slot u of a lane refers to x[j[u] * stride + col] (stride / col: the
 // interleaved columns of a multi-right-hand-side block; 1 / 0 otherwise).
 template <typename T, int U>
 __device__ __forceinline__ void await_batch(const T *x, const int (&j)[U], T (&xv)[U], int *err,
                                             int stride = 1, int col = 0) {
   x += col;
-  bool pend = false;
-#pragma unroll
-  for (int u = 0; u < U; u++)
-    if (j[u] >= 0 && Sent<T>::is(xv[u])) xv[u] = Sent<T>::load_agent(x + (size_t)j[u] * stride);
-#pragma unroll
-  for (int u = 0; u < U; u++) pend |= j[u] >= 0 && Sent<T>::is(xv[u]);
-  unsigned long long mask = __ballot(pend);
-  if (!mask) return;
   const int lane = __lane_id();
-  const long long t0 = wall_clock64();
-  int backoff = 1;
-  while (mask) {
+  for (unsigned long long mask = pending_lanes(j, xv); mask;) {
     const int leader = __ffsll((long long)mask) - 1;
     int jp = -1;
 #pragma unroll
     for (int u = U - 1; u >= 0; u--)
       if (j[u] >= 0 && Sent<T>::is(xv[u])) jp = j[u];
     jp = __shfl(jp, leader, 64);
-    if (lane == leader) {
-      for (int polls = 1;; polls++) {
-        if (kPollCap > 0)
-          for (int i = 0; i < backoff; i++) __builtin_amdgcn_s_sleep(1);
-        if (!Sent<T>::is(Sent<T>::load_agent(x + (size_t)jp * stride))) break;
-        if (backoff < kPollCap) backoff <<= 1;
-        if ((polls & 7) == 0 &&
-            (wall_clock64() - t0 > g_wait_ticks ||
-             __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
-          atomicOr(err, 1);
-          break;
-        }
-      }
-    }
-    backoff = 1;  // progress: the next wait is likely short
-    pend = false;
-#pragma unroll
-    for (int u = 0; u < U; u++)
-      if (j[u] >= 0 && Sent<T>::is(xv[u])) xv[u] = Sent<T>::load_agent(x + (size_t)j[u] * stride);
-#pragma unroll
-    for (int u = 0; u < U; u++) pend |= j[u] >= 0 && Sent<T>::is(xv[u]);
-    mask = __ballot(pend);
+    if (lane == leader) await_value(x + (size_t)jp * stride, err);
+    mask = reread_pending(x, j, xv, stride);
     if (mask && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-#pragma unroll
-      for (int u = 0; u < U; u++)
-        if (j[u] >= 0 && Sent<T>::is(xv[u])) xv[u] = T(0);
+      zero_pending(j, xv);
       break;
     }
   }
 }
 
-// Back-off cap of the all-lane phase of await_proxy, in s_sleep(1) units.
+// Back-off cap of await_all, in s_sleep(1) units.
 #ifndef RCHOL_AMD_POLL2_CAP
 #define RCHOL_AMD_POLL2_CAP 1
 #endif
 constexpr int kPoll2Cap = RCHOL_AMD_POLL2_CAP;
 
-// await_batch for a round whose wave knows a proxy: slot pu of lane pl
-// holds an entry a level or two below the latest of the round (the host's
-// choice), so once it is published the latest levels are being computed.  Phase 1: lane pl polls the proxy with back-off (one address,
-// however long the wait).  Phase 2: every lane re-reads its own pending
-// slots each poll, so a value is seen one load after its publication
-// instead of after a poll and a second, re-reading load.  The entries
-// still pending in phase 2 are few (most of a row's entries lie below the
-// latest level).  Same bound, error flag and zeroing as await_batch.
+// await_batch for a round whose proxy was published before it gathered: the
+// latest levels are being computed, few entries are pending, and every lane
+// re-reads its own each poll, so a value is seen one load after its
+// publication instead of after a poll and a second, re-reading load.  Same
+// bound, error flag and zeroing as await_batch.
 template <typename T, int U>
-__device__ __forceinline__ void await_proxy(const T *x, const int (&j)[U], T (&xv)[U], int *err,
-                                            int pl, int pu) {
-  bool pend = false;
-#pragma unroll
-  for (int u = 0; u < U; u++)
-    if (j[u] >= 0 && Sent<T>::is(xv[u])) xv[u] = Sent<T>::load_agent(x + j[u]);
-#pragma unroll
-  for (int u = 0; u < U; u++) pend |= j[u] >= 0 && Sent<T>::is(xv[u]);
-  unsigned long long mask = __ballot(pend);
-  if (!mask) return;
-  const int lane = __lane_id();
-  const long long t0 = wall_clock64();
-  int jp = -1, wait = 0;
-#pragma unroll
-  for (int u = 0; u < U; u++)
-    if (u == pu) {
-      jp = j[u];
-      wait = Sent<T>::is(xv[u]) ? 1 : 0;
-    }
-  jp = __shfl(jp, pl, 64);
-  wait = __shfl(wait, pl, 64);
-  if (wait && lane == pl) {
-    int backoff = 1;
-    for (int polls = 1;; polls++) {
-      for (int i = 0; i < backoff; i++) __builtin_amdgcn_s_sleep(1);
-      if (!Sent<T>::is(Sent<T>::load_agent(x + jp))) break;
-      if (backoff < kPollCap) backoff <<= 1;
-      if ((polls & 7) == 0 &&
-          (wall_clock64() - t0 > g_wait_ticks ||
-           __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
-        atomicOr(err, 1);
-        break;
-      }
-    }
-  }
-  int backoff = 1;
-  for (int polls = 1;; polls++) {
-    pend = false;
-#pragma unroll
-    for (int u = 0; u < U; u++)
-      if (j[u] >= 0 && Sent<T>::is(xv[u])) xv[u] = Sent<T>::load_agent(x + j[u]);
-#pragma unroll
-    for (int u = 0; u < U; u++) pend |= j[u] >= 0 && Sent<T>::is(xv[u]);
-    mask = __ballot(pend);
+__device__ __forceinline__ void await_all(const T *x, const int (&j)[U], T (&xv)[U], int *err) {
+  Poll w;
+  for (;;) {
+    const unsigned long long mask = reread_pending(x, j, xv);
     if (!mask) return;
-    if ((polls & 7) == 0 &&
-        (wall_clock64() - t0 > g_wait_ticks ||
-         __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
-      if (lane == __ffsll((long long)mask) - 1) atomicOr(err, 1);
-#pragma unroll
-      for (int u = 0; u < U; u++)
-        if (j[u] >= 0 && Sent<T>::is(xv[u])) xv[u] = T(0);
+    if (w.expired(err)) {
+      if (__lane_id() == __ffsll((long long)mask) - 1) atomicOr(err, 1);
+      zero_pending(j, xv);
       return;
     }
-    for (int i = 0; i < backoff; i++) __builtin_amdgcn_s_sleep(1);
-    if (backoff < kPoll2Cap) backoff <<= 1;
+    w.sleep(kPoll2Cap);
   }
 }
 
-// Sum over the L consecutive lanes of a row group (L a power of two <= 64).
-template <int L>
-__device__ __forceinline__ double group_sum(double v) {
-#pragma unroll
-  for (int off = L / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, L);
-  return v;
+// Sum over the L consecutive lanes of a row group (L a power of two <= 64),
+// in every lane.  The steps pair lanes 1, 2, 4, 8, 16 and 32 apart (equal
+// bits in both lanes of a pair, since the addition commutes): within 16 lanes
+// by DPP moves -- once the lanes of a quad hold one value, the mirror of 8
+// lanes is the exchange 4 apart, and the mirror of 16 the one 8 apart -- and
+// across them by the lane swaps of gfx950.  No step goes through the LDS
+// crossbar, which costs a wave that just saw its last value about 0.06 us per
+// step (64 lanes, FP64: six steps of two words).
+template <int CTRL>
+__device__ __forceinline__ int dpp_word(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
 }
-template <int L>
-__device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-  for (int off = L / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, L);
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __int_as_float(dpp_word<CTRL>(__float_as_int(v)));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  return __hiloint2double(dpp_word<CTRL>(__double2hiint(v)), dpp_word<CTRL>(__double2loint(v)));
+}
+// v of this lane plus v of the lane 16 (32) apart.
+__device__ __forceinline__ float add_16_apart(float v) {
+  const auto w = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+  return __int_as_float(w[0]) + __int_as_float(w[1]);
+}
+__device__ __forceinline__ float add_32_apart(float v) {
+  const auto w = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+  return __int_as_float(w[0]) + __int_as_float(w[1]);
+}
+__device__ __forceinline__ double add_16_apart(double v) {
+  const int h = __double2hiint(v), l = __double2loint(v);
+  const auto wh = __builtin_amdgcn_permlane16_swap(h, h, false, false);
+  const auto wl = __builtin_amdgcn_permlane16_swap(l, l, false, false);
+  return __hiloint2double(wh[0], wl[0]) + __hiloint2double(wh[1], wl[1]);
+}
+__device__ __forceinline__ double add_32_apart(double v) {
+  const int h = __double2hiint(v), l = __double2loint(v);
+  const auto wh = __builtin_amdgcn_permlane32_swap(h, h, false, false);
+  const auto wl = __builtin_amdgcn_permlane32_swap(l, l, false, false);
+  return __hiloint2double(wh[0], wl[0]) + __hiloint2double(wh[1], wl[1]);
+}
+template <int L, typename T>
+__device__ __forceinline__ T group_sum(T v) {
+  if (L >= 2) v += dpp_move<0xB1>(v);    // quad_perm [1, 0, 3, 2]
+  if (L >= 4) v += dpp_move<0x4E>(v);    // quad_perm [2, 3, 0, 1]
+  if (L >= 8) v += dpp_move<0x141>(v);   // mirror of 8 lanes
+  if (L >= 16) v += dpp_move<0x140>(v);  // mirror of 16 lanes
+  if (L >= 32) v = add_16_apart(v);
+  if (L >= 64) v = add_32_apart(v);
   return v;
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
+__device__ __forceinline__ double wave_sum(double v) { return group_sum<64>(v); }
+
+// s / d with the reciprocal of d formed beforehand, so that a wave that just
+// saw its last value is three dependent operations from its quotient instead
+// of a whole division: q = s rd corrected by its exact remainder, which is
+// s / d correctly rounded when rd is and nothing leaves the normal range
+// (Markstein's theorem).  Anything else -- a pivot outside [2^-b, 2^b], a
+// quotient that is zero, tiny, huge or not finite -- takes the division.
+template <typename T>
+struct QuotRange;
+template <>
+struct QuotRange<double> {
+  static constexpr double lo = 0x1p-400, hi = 0x1p400;
+};
+template <>
+struct QuotRange<float> {
+  static constexpr float lo = 0x1p-40f, hi = 0x1p40f;
+};
+__device__ __forceinline__ double fma_of(double a, double b, double c) { return __fma_rn(a, b, c); }
+__device__ __forceinline__ float fma_of(float a, float b, float c) { return __fmaf_rn(a, b, c); }
+__device__ __forceinline__ double abs_of(double a) { return fabs(a); }
+__device__ __forceinline__ float abs_of(float a) { return fabsf(a); }
+template <typename T>
+struct Divisor {
+  T d, rd;
+  bool plain;  // this lane divides
+  __device__ __forceinline__ explicit Divisor(T d_) : d(d_), rd(T(1) / d_) {
+    const T a = abs_of(rd);
+    plain = !(a > QuotRange<T>::lo && a < QuotRange<T>::hi);
+    asm volatile("" : "+v"(rd));  // formed here, before the waits
+  }
+  // s / d in the lanes that use it
+  __device__ __forceinline__ T quotient(T s, bool used) const {
+    const T q0 = s * rd;
+    const T q = fma_of(fma_of(-q0, d, s), rd, q0);
+    const T a = abs_of(q);
+    const bool slow = plain || !(a > QuotRange<T>::lo && a < QuotRange<T>::hi);
+    // a wave-uniform branch: otherwise the division is computed in every lane
+    if (__ballot(used && slow)) return slow ? s / d : q;
+    return q;
+  }
+};
 
 // Block-wide sum of NV doubles (blockDim.x a multiple of 64, <= 1024);
 // the result is valid in thread 0.  Deterministic for a fixed launch shape.

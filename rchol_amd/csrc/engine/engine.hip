@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -124,6 +125,8 @@ struct DevBuf {
   }
 };
 
+#include "analysis.hpp"
+
 // One triangular sweep on the device: rows in level ("slot") order.
 struct Sweep {
   int nslots = 0, ntasks = 0, nlevels = 0;
@@ -132,9 +135,18 @@ struct Sweep {
   // split schedule: levels [0, head_end) and [tail_begin, nlevels) run in one
   // workgroup (k_sptrsv_serial), the middle in the persistent kernel
   std::vector<int> level_ptr_h, rp_h;
-  std::vector<unsigned short> proxy_h;  // per slot: proxy distance (0: none)
+  IntVec proxy_h;  // per slot: its row's proxy (the row to wait for; -1: none)
+  // merged levels (merge_plan.hpp): groups of levels, the slots [m0, m1) whose
+  // rows may be merged; mrp is indexed by slot - m0
+  std::vector<int> gptr_h, mrp_h;
+  IntVec mproxy_h;  // proxies of the merged rows, by slot - m0
+  int m0 = 0, m1 = 0;
+  DevBuf<int> mrp, mci;
+  DevBuf<double> mcv64;
+  DevBuf<float> mcv32;
   DevBuf<int> level_ptr, level_lg;
-  DevBuf<int> wave_ptr, wt_s0, wt_info;  // middle tasks in per-wave lists
+  DevBuf<int> wave_ptr;  // middle tasks in per-wave lists
+  DevBuf<SweepTask> wt;
   int head_end = 0, tail_begin = 0, mid_ntasks = 0;
   DevBuf<double> cv64, diag64;
   DevBuf<float> cv32, diag32;
@@ -172,9 +184,9 @@ struct Sweep {
   } ch;
 };
 
-#include "analysis.hpp"
-
 #include "chunk_plan.hpp"
+
+#include "merge_plan.hpp"
 
 // Cut a sweep's levels into a narrow head, a middle and a narrow tail
 // (levels of at most `width` rows run in one workgroup; width 0 = no split).
@@ -210,61 +222,82 @@ int lane_lg(int len, int lmin_lg) {
 constexpr long long kWideRowsPerWave = RCHOL_AMD_WIDE_ROWS;  // stream-task threshold
 
 struct TaskCut {
-  std::vector<int> s0, info, level;  // info = cnt | lg << kTaskInfoShift
+  std::vector<int> s0, info, px, level;  // info = cnt | lane code << kTaskInfoShift
 };
 
-void cut_tasks(const std::vector<int> &lp, const std::vector<int> &rp,
-               const std::vector<unsigned short> &proxy, int h, int t, int lmin_lg,
-               long long nwaves, bool flat_ok, TaskCut &tc) {
+// Levels merged into one group (merge_plan.hpp) are one level here: the
+// rows of its first level as they are, the others in their merged form.  A
+// group that holds a wide level is cut level by level instead.
+void cut_tasks(const Sweep &sw, int h, int t, int lmin_lg, long long nwaves, bool flat_ok,
+               bool merge, TaskCut &tc) {
+  const std::vector<int> &lp = sw.level_ptr_h;
   tc.s0.clear();
   tc.info.clear();
+  tc.px.clear();
   tc.level.clear();
-  auto push = [&](int s, int cnt, int lg, int l) {
-    // a lane task's proxy: that of its first row that has one in the first
-    // round (one pass: row k is row group k)
-    int px = 0;
-    if (RCHOL_AMD_PROXY && lg < kTaskStream && (size_t)(s + cnt) <= proxy.size())
-      for (int k = 0; k < cnt; k++) {
-        const int pc = proxy[s + k];
-        if (pc > 0 && pc < (kGather << lg)) {
-          px = pc | (k << 9);
-          break;
-        }
-      }
+  auto push = [&](int s, int cnt, int lg, int l, int px = -1, int flag = 0) {
     tc.s0.push_back(s);
-    tc.info.push_back(cnt | (lg << kTaskInfoShift) | (px << kTaskProxyShift));
+    tc.info.push_back(cnt | (lg << kTaskInfoShift) | flag);
+    tc.px.push_back(px);
     tc.level.push_back(l);
   };
-  for (int l = h; l < t; l++) {
-    const int s_end = lp[l + 1];
-    const long long rows = s_end - lp[l];
-    const bool wide = rows > kWideRowsPerWave * nwaves;
-    if (flat_ok && wide && rp[s_end] == rp[lp[l]]) {  // a wide level that reads nothing
-      for (int s = lp[l]; s < s_end; s += 64 * kFlatPerLane)
-        push(s, std::min(s_end - s, 64 * kFlatPerLane), kTaskFlat, l);
-      continue;
-    }
-    for (int s = lp[l]; s < s_end;) {
-      if (wide) {
-        int k = 1;  // at least one row, however long (the kernel loops rounds)
-        while (s + k < s_end && k < 64 && rp[s + k + 1] - rp[s] <= 64 * kStream) k++;
-        push(s, k, kTaskStream, l);
-        s += k;
-        continue;
-      }
-      int lg = lane_lg(rp[s + 1] - rp[s], lmin_lg);
+  // lane tasks of slots [s, s_end): lg_of(slot) the least width that covers
+  // the slot's row in one round, px_of[slot] its proxy
+  auto cut_lanes = [&](int s, int s_end, int l, const int *px_of, int flag, auto &&lg_of) {
+    while (s < s_end) {
+      int lg = lg_of(s);
       for (;;) {  // widen until the longest of the 64/L rows fits one round
         const int take = std::min(s_end - s, 64 >> lg);
         int need = lg;
-        for (int k = 0; k < take; k++)
-          need = std::max(need, lane_lg(rp[s + k + 1] - rp[s + k], lmin_lg));
+        for (int k = 0; k < take; k++) need = std::max(need, lg_of(s + k));
         if (need == lg) break;
         lg = need;
       }
       const int take = std::min(s_end - s, 64 >> lg);
-      push(s, take, lg, l);
+      int px = -1;  // the task's proxy: that of its first row that has one
+      for (int k = 0; k < take && px < 0; k++) px = px_of[s + k];
+      push(s, take, lg, l, px, flag);
       s += take;
     }
+  };
+  const int *rp = sw.rp_h.data();
+  const int *proxy = sw.proxy_h.data();
+  const int *mrp = sw.mrp_h.data() - sw.m0;
+  auto plain_lg = [&](int s) { return lane_lg(rp[s + 1] - rp[s], lmin_lg); };
+  auto merged_lg = [&](int s) { return lane_lg(mrp[s + 1] - mrp[s], lmin_lg); };
+  auto wide = [&](int l) { return lp[l + 1] - lp[l] > kWideRowsPerWave * nwaves; };
+  auto cut_level = [&](int l) {
+    const int s_end = lp[l + 1];
+    if (!wide(l)) {
+      cut_lanes(lp[l], s_end, l, proxy, 0, plain_lg);
+      return;
+    }
+    if (flat_ok && rp[s_end] == rp[lp[l]]) {  // a wide level that reads nothing
+      for (int s = lp[l]; s < s_end; s += 64 * kFlatPerLane)
+        push(s, std::min(s_end - s, 64 * kFlatPerLane), kTaskFlat, l);
+      return;
+    }
+    for (int s = lp[l]; s < s_end;) {
+      int k = 1;  // at least one row, however long (the kernel loops rounds)
+      while (s + k < s_end && k < 64 && rp[s + k + 1] - rp[s] <= 64 * kStream) k++;
+      push(s, k, kTaskStream, l);
+      s += k;
+    }
+  };
+  if (!merge || sw.m1 == sw.m0) {
+    for (int l = h; l < t; l++) cut_level(l);
+    return;
+  }
+  for (size_t g = 0; g + 1 < sw.gptr_h.size(); g++) {
+    const int a = sw.gptr_h[g], b = sw.gptr_h[g + 1];
+    bool split = b - a == 1;
+    for (int l = a; l < b; l++) split |= wide(l);
+    if (split) {
+      for (int l = a; l < b; l++) cut_level(l);
+      continue;
+    }
+    cut_lanes(lp[a], lp[a + 1], a, proxy, 0, plain_lg);
+    cut_lanes(lp[a + 1], lp[b], a, sw.mproxy_h.data() - sw.m0, kTaskMerged, merged_lg);
   }
 }
 
@@ -277,6 +310,7 @@ void cut_tasks_mr(const std::vector<int> &lp, const std::vector<int> &rp, int nl
                   long long nwaves, TaskCut &tc) {
   tc.s0.clear();
   tc.info.clear();
+  tc.px.clear();
   tc.level.clear();
   int maxlg = 0;
   while ((K << (maxlg + 1)) <= 64) maxlg++;
@@ -299,6 +333,7 @@ void cut_tasks_mr(const std::vector<int> &lp, const std::vector<int> &rp, int nl
       }
       tc.s0.push_back(s);
       tc.info.push_back(take | (lg << kTaskInfoShift));
+      tc.px.push_back(-1);
       tc.level.push_back(l);
       s += take;
     }
@@ -313,7 +348,7 @@ void cut_tasks_mr(const std::vector<int> &lp, const std::vector<int> &rp, int nl
 // levels.  Each wave's list is in level order, which is all the
 // deadlock-freedom argument of k_sptrsv needs.
 void assign_waves(const TaskCut &tc, int nblocks, std::vector<int> &wave_ptr,
-                  std::vector<int> &ws0, std::vector<int> &winfo) {
+                  std::vector<SweepTask> &wt) {
   const int W = nblocks * 4;
   const int X = nblocks >= 8 ? 8 : 1;
   std::vector<std::vector<int>> xw(X);  // waves of each XCD
@@ -334,19 +369,12 @@ void assign_waves(const TaskCut &tc, int nblocks, std::vector<int> &wave_ptr,
     i = j;
   }
   wave_ptr.assign(W + 1, 0);
-  ws0.clear();
-  winfo.clear();
+  wt.clear();
   for (int w = 0; w < W; w++) {
-    for (int k : lists[w]) {
-      ws0.push_back(tc.s0[k]);
-      winfo.push_back(tc.info[k]);
-    }
-    wave_ptr[w + 1] = (int)ws0.size();
+    for (int k : lists[w]) wt.push_back({tc.s0[k], tc.info[k], tc.px[k], 0});
+    wave_ptr[w + 1] = (int)wt.size();
   }
-  if (ws0.empty()) {
-    ws0.push_back(0);
-    winfo.push_back(0);
-  }
+  if (wt.empty()) wt.push_back({0, 0, -1, 0});
 }
 
 // Upload a sweep's split schedule: head/tail bounds [0, h) / [t, nlevels),
@@ -364,12 +392,12 @@ hipError_t upload_schedule(Sweep &sw, int h, int t, int lmin_lg, const TaskCut &
   sw.head_end = h;
   sw.tail_begin = t;
   sw.mid_ntasks = (int)tc.s0.size();
-  std::vector<int> wp, ws0, winfo;
-  assign_waves(tc, nblocks, wp, ws0, winfo);
+  std::vector<int> wp;
+  std::vector<SweepTask> wt;
+  assign_waves(tc, nblocks, wp, wt);
   hipError_t e = sw.level_lg.upload(llg.data(), llg.size());
   if (e == hipSuccess) e = sw.wave_ptr.upload(wp.data(), wp.size());
-  if (e == hipSuccess) e = sw.wt_s0.upload(ws0.data(), ws0.size());
-  if (e == hipSuccess) e = sw.wt_info.upload(winfo.data(), winfo.size());
+  if (e == hipSuccess) e = sw.wt.upload(wt.data(), wt.size());
   return e;
 }
 
@@ -415,6 +443,7 @@ struct rchol_amd_ctx {
   int task_waves = 0;       // waves the task cut plans for (0 = resident capacity)
   int strict_sync = 0;      // grid reductions with release/acquire fences
   int chunk_mode = -1;      // RCHOL_AMD_OPT_CHUNKED
+  int merge_levels = 1;     // RCHOL_AMD_OPT_MERGE
   bool chunk_auto = false;  // the upload's own choice (chunk_mode -1)
   bool use_chunks = false;  // single-RHS sweeps run k_sptrsv_chunk
   int lds_max = 0;          // LDS bytes a workgroup may allocate
@@ -439,7 +468,8 @@ struct rchol_amd_ctx {
     hipGraphExec_t gexec = nullptr;
     int grid = 0;
     // sweep schedule cut for K columns: per-wave task lists, [0] fwd, [1] bwd
-    DevBuf<int> wave_ptr[2], wt_s0[2], wt_info[2];
+    DevBuf<int> wave_ptr[2];
+    DevBuf<SweepTask> wt[2];
     int sched_K = 0, ntasks[2] = {0, 0};
     long long sched_gen = -1;
     void drop_graph() {
@@ -555,6 +585,9 @@ void launch_one_sweep(rchol_amd_ctx *c, const Sweep &sw, const VT *cv, const VT 
                        stop);
     return;
   }
+  const VT *mcv;
+  if constexpr (sizeof(VT) == 8) mcv = sw.mcv64.p; else mcv = sw.mcv32.p;
+  const int *mrp = sw.mrp.p ? sw.mrp.p - sw.m0 : nullptr;  // indexed by slot
   const bool head = sw.head_end > 0, tail = sw.tail_begin < sw.nlevels;
   if (head)
     hipLaunchKernelGGL((k_sptrsv_serial<VT, XT, BT, FUSE>), dim3(1), dim3(1024), 0, c->stream, 0,
@@ -562,9 +595,9 @@ void launch_one_sweep(rchol_amd_ctx *c, const Sweep &sw, const VT *cv, const VT 
                        sw.ci.p, cv, dg, rhs, x, aux, dotv, sc, stop, 0);
   if (sw.mid_ntasks > 0 || (FUSE == 2 && !tail))
     hipLaunchKernelGGL((k_sptrsv<VT, XT, BT, FUSE>), dim3(c->trsv_grid), dim3(kBlock), 0,
-                       c->stream, sw.wave_ptr.p, sw.wt_s0.p, sw.wt_info.p,
-                       sw.slot_row.p, sw.rp.p, sw.ci.p, cv, dg, rhs, x, aux, dotv, c->partials.p,
-                       sc, stop, tail ? 1 : 0, c->coherent_gather);
+                       c->stream, sw.wave_ptr.p, sw.wt.p,
+                       sw.slot_row.p, sw.rp.p, sw.ci.p, cv, mrp, (const int *)sw.mci.p, mcv, dg, rhs, x, aux, dotv, c->partials.p, sc, stop, tail ? 1 : 0,
+                       c->coherent_gather);
   if (tail)
     hipLaunchKernelGGL((k_sptrsv_serial<VT, XT, BT, FUSE>), dim3(1), dim3(1024), 0, c->stream,
                        sw.tail_begin, sw.nlevels, sw.level_ptr.p, sw.level_lg.p, sw.slot_row.p,
@@ -700,8 +733,7 @@ int rchol_amd_ctx::size_trsv_grid() {
   size_t max_tasks = 0;
   for (int k = 0; k < 2; k++) {
     compute_split(sw[k]->level_ptr_h, sw[k]->nlevels, serial_width, h[k], t[k]);
-    cut_tasks(sw[k]->level_ptr_h, sw[k]->rp_h, sw[k]->proxy_h, h[k], t[k], lmin_lg, plan_waves,
-              k == 0, tc[k]);
+    cut_tasks(*sw[k], h[k], t[k], lmin_lg, plan_waves, k == 0, serial_width == 0, tc[k]);
     max_tasks = std::max(max_tasks, tc[k].s0.size());
   }
   trsv_grid = (int)std::max<size_t>(1, std::min<size_t>(cap_blocks, (max_tasks + 3) / 4));
@@ -966,11 +998,11 @@ int rchol_amd_ctx::ensure_batch_schedule(int K, int per_cu) {
   batch.grid = (int)std::max<size_t>(1, std::min<size_t>(cap_blocks, (max_tasks + 3) / 4));
   HIP_TRY(hipMemset(&batch.bs->arrive, 0, sizeof(batch.bs->arrive)));
   for (int k = 0; k < 2; k++) {
-    std::vector<int> wp, ws0, winfo;
-    assign_waves(tc[k], batch.grid, wp, ws0, winfo);
+    std::vector<int> wp;
+    std::vector<SweepTask> wt;
+    assign_waves(tc[k], batch.grid, wp, wt);
     HIP_TRY(batch.wave_ptr[k].upload(wp.data(), wp.size()));
-    HIP_TRY(batch.wt_s0[k].upload(ws0.data(), ws0.size()));
-    HIP_TRY(batch.wt_info[k].upload(winfo.data(), winfo.size()));
+    HIP_TRY(batch.wt[k].upload(wt.data(), wt.size()));
     batch.ntasks[k] = (int)tc[k].s0.size();
   }
   batch.sched_K = K;
@@ -982,36 +1014,30 @@ template <int K>
 void rchol_amd_ctx::launch_sweeps_mr(const double *rhs, bool with_dot, const int *stop,
                                      hipEvent_t *ev) {
   const dim3 g(batch.grid), blk(kBlock);
-  const int *wpf = batch.wave_ptr[0].p, *wsf = batch.wt_s0[0].p, *wif = batch.wt_info[0].p;
-  const int *wpb = batch.wave_ptr[1].p, *wsb = batch.wt_s0[1].p, *wib = batch.wt_info[1].p;
+  const int *wpf = batch.wave_ptr[0].p, *wpb = batch.wave_ptr[1].p;
+  const SweepTask *wtf = batch.wt[0].p, *wtb = batch.wt[1].p;
   if (gprec == RCHOL_AMD_FP32) {
-    hipLaunchKernelGGL((k_sptrsv_mr<float, float, double, K, 1>), g, blk, 0, stream, wpf, wsf,
-                       wif, fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv32.p, fwd.diag32.p, rhs,
+    hipLaunchKernelGGL((k_sptrsv_mr<float, float, double, K, 1>), g, blk, 0, stream, wpf, wtf, fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv32.p, fwd.diag32.p, rhs,
                        batch.y32.p, batch.z32.p, nullptr, nullptr, batch.bs, stop);
     if (ev) (void)hipEventRecord(ev[1], stream);
     if (with_dot)
-      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 2>), g, blk, 0, stream, wpb, wsb,
-                         wib, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, bwd.diag32.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 2>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, bwd.diag32.p,
                          (const float *)batch.y32.p, batch.z32.p, (float *)nullptr,
                          (const double *)batch.r.p, batch.partials.p, batch.bs, stop);
     else
-      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 0>), g, blk, 0, stream, wpb, wsb,
-                         wib, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, bwd.diag32.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 0>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, bwd.diag32.p,
                          (const float *)batch.y32.p, batch.z32.p, (float *)nullptr, nullptr,
                          nullptr, batch.bs, stop);
   } else {
-    hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 1>), g, blk, 0, stream, wpf, wsf,
-                       wif, fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv64.p, fwd.diag64.p, rhs,
+    hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 1>), g, blk, 0, stream, wpf, wtf, fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv64.p, fwd.diag64.p, rhs,
                        batch.y64.p, batch.z64.p, nullptr, nullptr, batch.bs, stop);
     if (ev) (void)hipEventRecord(ev[1], stream);
     if (with_dot)
-      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 2>), g, blk, 0, stream, wpb,
-                         wsb, wib, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, bwd.diag64.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 2>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, bwd.diag64.p,
                          (const double *)batch.y64.p, batch.z64.p, (double *)nullptr,
                          (const double *)batch.r.p, batch.partials.p, batch.bs, stop);
     else
-      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 0>), g, blk, 0, stream, wpb,
-                         wsb, wib, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, bwd.diag64.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 0>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, bwd.diag64.p,
                          (const double *)batch.y64.p, batch.z64.p, (double *)nullptr, nullptr,
                          nullptr, batch.bs, stop);
   }
@@ -1701,6 +1727,13 @@ int chunk_launch_setup(rchol_amd_ctx *c, size_t lds) {
   return RCHOL_AMD_OK;
 }
 
+// Whether the upload plans the chunked sweeps.
+bool plans_chunks(const rchol_amd_ctx *c, size_t n, int nlf, int nlb) {
+  const int nl = std::max(nlf, nlb);
+  const bool deep = nl >= kChunkMinLevels && (double)n / nl < kChunkMaxMeanWidth;
+  return c->chunk_mode == 1 || (c->chunk_mode == -1 && deep);
+}
+
 // Plan (and, when chosen, upload) the chunked sweeps of a factor whose
 // analysis is in hf / hb.
 int setup_chunks(rchol_amd_ctx *c, size_t n, HostSweep &hf, HostSweep &hb, int nlf,
@@ -1709,9 +1742,7 @@ int setup_chunks(rchol_amd_ctx *c, size_t n, HostSweep &hf, HostSweep &hb, int n
   c->bwd.ch.reset();
   c->use_chunks = false;
   c->chunk_auto = false;
-  const int nl = std::max(nlf, nlb);
-  const bool deep = nl >= kChunkMinLevels && (double)n / nl < kChunkMaxMeanWidth;
-  if (!(c->chunk_mode == 1 || (c->chunk_mode == -1 && deep))) return RCHOL_AMD_OK;
+  if (!plans_chunks(c, n, nlf, nlb)) return RCHOL_AMD_OK;
   const size_t xt = precision == RCHOL_AMD_FP32 ? sizeof(float) : sizeof(double);
   const size_t budget = c->lds_max > 2048 ? (size_t)c->lds_max - 1024 : 0;
   const int S = (int)std::min<size_t>(kChunkMaxRows, budget / xt - 1);
@@ -1763,6 +1794,29 @@ int rchol_amd_upload_G(rchol_amd_ctx *c, size_t n, const size_t *colPtr, const s
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->drop_graph();
   c->hasG = false;
+  // the merge plans are made while the plain rows go to the device
+  MergePlan mplan[2];
+  std::thread planner;
+  struct Join {
+    std::thread &t;
+    ~Join() {
+      if (t.joinable()) t.join();
+    }
+  } join{planner};
+  if (c->merge_levels && !plans_chunks(c, n, nlf, nlb)) {
+    auto plan = [&]() {
+      for (int k = 0; k < 2; k++) try {
+          plan_merge(k ? hb : hf, n, mplan[k]);
+        } catch (const std::exception &) {  // no memory or threads for it: the plain levels
+          mplan[k] = MergePlan();
+        }
+    };
+    try {
+      planner = std::thread(plan);
+    } catch (const std::exception &) {
+      plan();
+    }
+  }
   auto up = [&](Sweep &sw, HostSweep &h) -> int {
     sw.nslots = (int)n;
     sw.ntasks = (int)h.task_ptr.size() - 1;
@@ -1771,7 +1825,12 @@ int rchol_amd_upload_G(rchol_amd_ctx *c, size_t n, const size_t *colPtr, const s
     HIP_TRY(sw.task_ptr.upload(h.task_ptr.data(), h.task_ptr.size()));
     sw.level_ptr_h = h.level_ptr;
     sw.rp_h.assign(h.rp.begin(), h.rp.end());
-    sw.proxy_h.assign(h.proxy.begin(), h.proxy.end());
+    sw.proxy_h.resize(n);  // the proxies as rows to wait for
+    par_for(n, [&](size_t s0, size_t s1) {
+      for (size_t s = s0; s < s1; s++)
+        sw.proxy_h[s] =
+            h.proxy[s] ? h.nat_ci[h.nat_rp[(size_t)h.slot_row[s] + 1] - 1 - h.proxy[s]] : -1;
+    });
     HIP_TRY(sw.level_ptr.upload(h.level_ptr.data(), h.level_ptr.size()));
     HIP_TRY(sw.slot_row.upload(h.slot_row.data(), n));
     HIP_TRY(sw.rp.upload(h.rp.data(), n + 1));
@@ -1784,11 +1843,33 @@ int rchol_amd_upload_G(rchol_amd_ctx *c, size_t n, const size_t *colPtr, const s
     HIP_TRY(sw.ci.alloc(noff));
     return precision == RCHOL_AMD_FP32 ? gather_slots<float>(c, sw, h, sw.cv32, sw.diag32)
                                        : gather_slots<double>(c, sw, h, sw.cv64, sw.diag64);
+  };
+  auto up_merged = [&](Sweep &sw, MergePlan &mp) -> int {
+    sw.m0 = mp.m0;
+    sw.m1 = mp.m1;
+    sw.gptr_h = std::move(mp.gptr);
+    sw.mrp_h.assign(mp.rp.begin(), mp.rp.end());
+    sw.mproxy_h.resize(mp.proxy.size());
+    for (size_t k = 0; k < mp.proxy.size(); k++)
+      sw.mproxy_h[k] = mp.proxy[k] ? mp.ci[mp.rp[k + 1] - 1 - mp.proxy[k]] : -1;
+    sw.mrp.reset();
+    sw.mci.reset();
+    sw.mcv64.reset();
+    sw.mcv32.reset();
+    if (sw.m1 == sw.m0) return RCHOL_AMD_OK;
+    HIP_TRY(sw.mrp.upload(mp.rp.data(), mp.rp.size()));
+    HIP_TRY(sw.mci.upload(mp.ci.data(), mp.ci.size()));
+    if (precision == RCHOL_AMD_FP32)
+      HIP_TRY(upload_as(sw.mcv32, mp.cv));
+    else
+      HIP_TRY(upload_as(sw.mcv64, mp.cv));
     return RCHOL_AMD_OK;
   };
   int rc = up(c->fwd, hf);
-  if (rc) return rc;
-  rc = up(c->bwd, hb);
+  if (!rc) rc = up(c->bwd, hb);
+  if (planner.joinable()) planner.join();
+  if (!rc) rc = up_merged(c->fwd, mplan[0]);
+  if (!rc) rc = up_merged(c->bwd, mplan[1]);
   if (rc) return rc;
   c->nG = n;
   c->nnzG = nnz;
@@ -1842,6 +1923,9 @@ int rchol_amd_set_option(rchol_amd_ctx *c, int key, double value) {
       break;
     case RCHOL_AMD_OPT_COHERENT_GATHER:
       c->coherent_gather = v ? 1 : 0;
+      break;
+    case RCHOL_AMD_OPT_MERGE:
+      c->merge_levels = v ? 1 : 0;
       break;
     case RCHOL_AMD_OPT_STRICT_SYNC:
       c->strict_sync = v ? 1 : 0;
@@ -2522,6 +2606,33 @@ int rchol_amd_chunk_apply_host(size_t n, const size_t *colPtr, const size_t *row
   return RCHOL_AMD_OK;
 }
 
+int rchol_amd_merge_apply_host(size_t n, const size_t *colPtr, const size_t *rowIdx,
+                               const double *val, const double *r, double *z, int *groups,
+                               long long *entries, double *est_us) {
+  if (!colPtr || !rowIdx || !val || !r || !z) return fail(RCHOL_AMD_EINVAL, "null argument");
+  if (n == 0 || n > kIdxMax) return fail(RCHOL_AMD_ERANGE, "n=%zu outside [1, 2^31)", n);
+  if (colPtr[0] != 0) return fail(RCHOL_AMD_EINVAL, "colPtr[0] must be 0");
+  if (colPtr[n] > kIdxMax) return fail(RCHOL_AMD_ERANGE, "nnz(G) exceeds the int32 index range");
+  HostSweep hf, hb;
+  int nlf = 0, nlb = 0;
+  int rc = analyze_factor(n, colPtr, rowIdx, val, hf, hb, nlf, nlb);
+  if (rc) return rc;
+  MergePlan pf, pb;
+  plan_merge(hf, n, pf);
+  plan_merge(hb, n, pb);
+  std::vector<double> y(n);
+  rc = simulate_merge(hf, pf, n, r, y.data());
+  if (!rc) rc = simulate_merge(hb, pb, n, y.data(), z);
+  if (rc) return rc;
+  const MergePlan *p[2] = {&pf, &pb};
+  for (int k = 0; k < 2; k++) {
+    if (groups) groups[k] = p[k]->any() ? (int)p[k]->gptr.size() - 1 : (k ? nlb : nlf);
+    if (entries) entries[k] = (long long)p[k]->ci.size();
+    if (est_us) est_us[k] = p[k]->est_us;
+  }
+  return RCHOL_AMD_OK;
+}
+
 void rchol_amd_schedule_free(rchol_amd_schedule *s) {
   if (!s) return;
   for (int k = 0; k < 2; k++) {
@@ -2541,6 +2652,7 @@ int rchol_amd_pcg_csr(size_t n, const size_t *aRowPtr, const size_t *aColIdx, co
   rchol_amd_ctx *c = nullptr;
   int rc = rchol_amd_create(0, &c);
   if (rc) return rc;
+  c->merge_levels = 0;  // one solve does not earn the plan back
   rc = rchol_amd_upload_A(c, n, aRowPtr, aColIdx, aVal);
   if (!rc) rc = rchol_amd_upload_G(c, n, gColPtr, gRowIdx, gVal, RCHOL_AMD_FP64);
   if (!rc) rc = rchol_amd_pcg(c, b, tol, maxit, x, x_in_is_initial, relres, itr);

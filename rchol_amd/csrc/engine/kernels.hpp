@@ -11,15 +11,17 @@ namespace rchol_amd {
 // ---------------------------------------------------------------------------
 // Sparse triangular sweep, pull form, persistent and level-scheduled.
 //
-// Rows are stored in "slot" order: sorted by dependency level (and inside a
-// level by decreasing length), so a slot range of one level holds mutually
-// independent rows.  The host cuts each level into tasks of at most 64
-// slots.  A task either has a lane width L = 2^lg (lg in [0, 6]) from the
-// length of its longest row, or -- rows of a wide level -- is a stream task
-// (sweep_stream).  The host gives every wave a static list of tasks in
-// level order (wave_ptr / wt_s0 / wt_info; no atomics).  A row reads x[j] of its dependencies; unpublished
-// entries still hold the sentinel and are polled until the producing wave
-// stores the value (agent-scope atomic store).  Deadlock freedom: every
+// Rows are stored in "slot" order: sorted by dependency level, so a slot
+// range of one level holds mutually independent rows; consecutive narrow
+// levels are merged into groups (merge_plan.hpp), whose rows are mutually
+// independent in their merged form.  The host cuts each level or group into
+// tasks: lane tasks (at most 64 / L rows of L = 2^lg lanes each, lg in [0, 6]
+// from the length of the longest row: sweep_lanes) or, for the rows of a wide
+// level, stream tasks (sweep_stream) and flat tasks (sweep_flat).  The host
+// gives every wave a static list of tasks in level order (wave_ptr / wt; no
+// atomics).  A row reads x[j] of its dependencies; unpublished entries still
+// hold the sentinel and are polled until the producing wave stores the value
+// (agent-scope atomic store).  Deadlock freedom: every
 // launched wave is resident (the grid is sized from the occupancy query),
 // each wave walks its list in level order and a task only depends on rows
 // of lower levels, so among the unfinished tasks of the lowest level, the
@@ -48,22 +50,39 @@ constexpr int kGather = RCHOL_AMD_GATHER;  // gathers in flight per lane and rou
 #define RCHOL_AMD_PROXY 1
 #endif
 
-// Sum of val[e] * x[ci[e]] over the entries e1 - 1 - sub - k L >= e0 of one
-// row, waiting for unpublished x.  The row is read from its end: its entries
-// are stored latest dependency last, so slot 0 of the first round -- the one
-// await_batch polls -- holds the value produced last.  Wave-converged call
-// (every lane of the wave, e0 == e1 for idle groups).
+// Per-slot metadata of a task, lane k holding slot s0 + k.
+template <typename VT>
+struct RowMeta {
+  int row = 0, e0 = 0, e1 = 0;
+  VT dg = 1;
+};
+
+// Sum of val[e] * x[ci[e]] over the entries [e0, e1) of one row, waiting for
+// unpublished x.  The row's entries are stored latest dependency last, and
+// its rounds are aligned to its end: slot 0 of the last round -- the one
+// await_batch polls -- holds the value produced last.  Earlier rounds (rows
+// of more than kGather * L entries) run first: their values are the oldest,
+// so only the last round usually waits.  Wave-converged call (every lane of
+// the wave, e0 == e1 for idle groups).
 //
-// px = pc | g << 9 with pc > 0: the first round holds a proxy
-// (await_proxy) at distance pc from the end of the row of row group g, i.e.
-// in lane g L + pc % L, slot pc / L; the task cut only sets it when
-// pc < kGather * L.
-template <typename VT, typename XT, int L, bool WAIT>
+// merged: the row may also hold right-hand sides of its own level group
+// (column c stored as -2 - c; see merge_plan.hpp), gathered from rhs.
+//
+// px >= 0: the row whose value the last round waits for before it gathers (a
+// proxy of its latest dependencies, see row_proxy).  A wave is usually at
+// its task long before its inputs are: gathering them then, and again once
+// they are there, loads the fabric that the publications travel on (128^3:
+// both sweeps of a merged factor 0.88 ms with the gather first, 0.84 ms
+// after the proxy).
+template <typename VT, typename XT, typename BT, int L>
 __device__ __forceinline__ XT row_dot(int e0, int e1, int sub, const int *__restrict__ ci,
-                                      const VT *__restrict__ cv, const XT *x, int *err,
-                                      int coherent, int px = 0) {
+                                      const VT *__restrict__ cv, const XT *x,
+                                      const BT *__restrict__ rhs, int *err, int coherent,
+                                      bool merged, int px) {
   XT acc = 0;
-  for (int c = e1 - 1 - sub; c >= e0; c -= kGather * L) {
+  constexpr int kRound = kGather * L;
+  for (int r = (e1 - e0 + kRound - 1) / kRound - 1; r >= 0; r--) {
+    const int c = e1 - 1 - sub - r * kRound;
     int j[kGather];
     VT v[kGather];
     XT xv[kGather];
@@ -73,27 +92,35 @@ __device__ __forceinline__ XT row_dot(int e0, int e1, int sub, const int *__rest
       j[u] = e >= e0 ? ld_stream(ci + e) : -1;
       v[u] = e >= e0 ? ld_stream(cv + e) : VT(0);
     }
+    const bool proxy = RCHOL_AMD_PROXY && px >= 0 && r == 0;
+    if (proxy) await_value(x + px, err);
 #pragma unroll
     for (int u = 0; u < kGather; u++) {
       if (j[u] < 0)
         xv[u] = XT(0);
-      else if (WAIT && coherent)
+      else if (coherent)
         xv[u] = Sent<XT>::load_agent(x + j[u]);
       else
         xv[u] = x[j[u]];
     }
-    if (WAIT) {
-      bool pend = false;
+    if (merged) {
+      bool tag = false;
 #pragma unroll
-      for (int u = 0; u < kGather; u++) pend |= Sent<XT>::is(xv[u]);
-      if (__ballot(pend)) {
-        const int pc = px & 511;
-        if (RCHOL_AMD_PROXY && pc > 0)
-          await_proxy<XT, kGather>(x, j, xv, err, (px >> 9) * L + pc % L, pc / L);
-        else
-          await_batch<XT, kGather>(x, j, xv, err);
+      for (int u = 0; u < kGather; u++) tag |= j[u] < -1;
+      if (__ballot(tag)) {
+        BT bv[kGather];
+#pragma unroll
+        for (int u = 0; u < kGather; u++) bv[u] = j[u] < -1 ? rhs[-2 - j[u]] : (BT)0;
+#pragma unroll
+        for (int u = 0; u < kGather; u++)
+          if (j[u] < -1) xv[u] = (XT)bv[u];
       }
-      px = 0;  // later rounds: entries of lower levels
+    }
+    if (pending_lanes(j, xv)) {
+      if (proxy)
+        await_all<XT, kGather>(x, j, xv, err);
+      else
+        await_batch<XT, kGather>(x, j, xv, err);
     }
 #pragma unroll
     for (int u = 0; u < kGather; u++) acc += (XT)v[u] * xv[u];
@@ -101,33 +128,33 @@ __device__ __forceinline__ XT row_dot(int e0, int e1, int sub, const int *__rest
   return acc;
 }
 
-// The rows of one task (cnt <= 64 slots, metadata already in lane k of the
-// m_* registers for slot k) with row groups of L lanes.
+// The rows of a lane task: cnt <= 64 / L slots, row group g of L lanes the
+// g-th.
 template <typename VT, typename XT, typename BT, int L, int FUSE>
-__device__ __forceinline__ void sweep_task(int cnt, int m_row, int m_e0, int m_e1, VT m_dg,
-                                           const int *__restrict__ ci, const VT *__restrict__ cv,
-                                           const BT *__restrict__ rhs, XT *x,
-                                           XT *__restrict__ aux, const double *__restrict__ dotv,
-                                           int *err, int coherent, double &dacc, int px) {
-  constexpr int R = 64 / L;
+__device__ __forceinline__ void sweep_lanes(int cnt, const RowMeta<VT> &m,
+                                            const int *__restrict__ ci, const VT *__restrict__ cv,
+                                            const BT *__restrict__ rhs, XT *x,
+                                            XT *__restrict__ aux, const double *__restrict__ dotv,
+                                            int *err, int coherent, double &dacc, bool merged,
+                                            int px) {
   const int lane = threadIdx.x & 63;
   const int grp = lane / L, sub = lane % L;
-  for (int base = 0; base < cnt; base += R) {
-    const int k = base + grp;  // < 64: base <= cnt - 1 - ((cnt - 1) % R)
-    const int row = __shfl(m_row, k, 64);
-    int e0 = __shfl(m_e0, k, 64), e1 = __shfl(m_e1, k, 64);
-    const VT dg = __shfl(m_dg, k, 64);
-    const bool live = k < cnt;
-    if (!live) e1 = e0;
-    const BT b = (live && sub == 0) ? ld_stream(rhs + row) : (BT)0;
-    XT acc = row_dot<VT, XT, L, true>(e0, e1, sub, ci, cv, x, err, coherent, base == 0 ? px : 0);
-    acc = group_sum<L>(acc);
-    if (live && sub == 0) {
-      const XT v = ((XT)b - acc) / (XT)dg;
-      Sent<XT>::store_agent(x + row, v);
-      if (FUSE == 1) aux[row] = Sent<XT>::value();
-      if (FUSE == 2) dacc += dotv[row] * (double)v;
-    }
+  const int row = __shfl(m.row, grp, 64);
+  int e0 = __shfl(m.e0, grp, 64), e1 = __shfl(m.e1, grp, 64);
+  const Divisor<XT> div((XT)__shfl(m.dg, grp, 64));
+  const bool live = grp < cnt;
+  if (!live) e1 = e0;
+  const bool writes = live && sub == 0;
+  // before the waits: what the epilogue needs besides the sum
+  const BT b = writes ? ld_stream(rhs + row) : (BT)0;
+  const double dv = FUSE == 2 && writes ? dotv[row] : 0.0;
+  XT acc = row_dot<VT, XT, BT, L>(e0, e1, sub, ci, cv, x, rhs, err, coherent, merged, px);
+  acc = group_sum<L>(acc);
+  const XT v = div.quotient((XT)b - acc, writes);
+  if (writes) {
+    Sent<XT>::store_agent(x + row, v);
+    if (FUSE == 1) aux[row] = Sent<XT>::value();
+    if (FUSE == 2) dacc += dv * (double)v;
   }
 }
 
@@ -146,7 +173,13 @@ constexpr int kTaskStream = 7;             // lane code of a stream task
 constexpr int kTaskFlat = 8;               // lane code of a flat task (see sweep_flat)
 constexpr int kFlatPerLane = 8;            // slots per lane of a flat task
 constexpr int kTaskInfoShift = 10;         // task info word: slot count | lane code << 10
-constexpr int kTaskProxyShift = 14;        //   | proxy (lane tasks: distance | row group << 9) << 14
+constexpr int kTaskMerged = 1 << 14;       //   | the rows of a lane task are merged rows
+
+// A task of a wave's list: first slot, info word, proxy (lane tasks: the row
+// to wait for before gathering, -1: none).
+struct alignas(16) SweepTask {
+  int s0, info, px, pad;
+};
 
 // acc + buf[lo] + buf[lo + 1] + ... + buf[hi - 1], added in that order, with
 // four LDS reads in flight at a time (a plain loop waits for each read).
@@ -165,7 +198,7 @@ __device__ __forceinline__ T lds_row_sum(const T *buf, int lo, int hi, T acc) {
 }
 
 template <typename VT, typename XT, typename BT, int FUSE>
-__device__ __forceinline__ void sweep_stream(int cnt, int m_row, int m_e0, int m_e1, VT m_dg,
+__device__ __forceinline__ void sweep_stream(int cnt, const RowMeta<VT> &m,
                                              const int *__restrict__ ci,
                                              const VT *__restrict__ cv,
                                              const BT *__restrict__ rhs, XT *x,
@@ -174,8 +207,11 @@ __device__ __forceinline__ void sweep_stream(int cnt, int m_row, int m_e0, int m
                                              int coherent, double &dacc, XT *buf) {
   const int lane = threadIdx.x & 63;
   const bool live = lane < cnt;
+  const int m_row = m.row, m_e0 = m.e0, m_e1 = m.e1;
+  const VT m_dg = m.dg;
   const int E0 = __shfl(m_e0, 0, 64), E1 = __shfl(m_e1, cnt - 1, 64);
   const BT b = live ? ld_stream(rhs + m_row) : (BT)0;
+  const double dv = FUSE == 2 && live ? dotv[m_row] : 0.0;
   XT acc = 0;
   for (int c = E0; c < E1; c += 64 * kStream) {
     int j[kStream];
@@ -196,10 +232,7 @@ __device__ __forceinline__ void sweep_stream(int cnt, int m_row, int m_e0, int m
       else
         xv[u] = x[j[u]];
     }
-    bool pend = false;
-#pragma unroll
-    for (int u = 0; u < kStream; u++) pend |= Sent<XT>::is(xv[u]);
-    if (__ballot(pend)) await_batch<XT, kStream>(x, j, xv, err);
+    if (pending_lanes(j, xv)) await_batch<XT, kStream>(x, j, xv, err);
 #pragma unroll
     for (int u = 0; u < kStream; u++) buf[u * 64 + lane] = (XT)v[u] * xv[u];
     // LDS requests of one wave complete in order; the fences only keep the
@@ -219,7 +252,7 @@ __device__ __forceinline__ void sweep_stream(int cnt, int m_row, int m_e0, int m
     const XT r = ((XT)b - acc) / (XT)m_dg;
     Sent<XT>::store_agent(x + m_row, r);
     if (FUSE == 1) aux[m_row] = Sent<XT>::value();
-    if (FUSE == 2) dacc += dotv[m_row] * (double)r;
+    if (FUSE == 2) dacc += dv * (double)r;
   }
 }
 
@@ -258,15 +291,15 @@ __device__ __forceinline__ void sweep_flat(int s0, int cnt, const int *__restric
 
 template <typename VT, typename XT, typename BT, int FUSE>
 __global__ __launch_bounds__(256) void k_sptrsv(
-    const int *__restrict__ wave_ptr, const int *__restrict__ wt_s0,
-    const int *__restrict__ wt_info, const int *__restrict__ slot_row,
-    const int *__restrict__ rp, const int *__restrict__ ci, const VT *__restrict__ cv,
-    const VT *__restrict__ diag, const BT *__restrict__ rhs, XT *x, XT *__restrict__ aux,
-    const double *__restrict__ dotv, double *__restrict__ partials, DevScalars *sc,
-    const int *stop, int defer, int coherent) {
+    const int *__restrict__ wave_ptr, const SweepTask *__restrict__ wt,
+    const int *__restrict__ slot_row, const int *__restrict__ rp, const int *__restrict__ ci,
+    const VT *__restrict__ cv, const int *__restrict__ mrp, const int *__restrict__ mci,
+    const VT *__restrict__ mcv, const VT *__restrict__ diag, const BT *__restrict__ rhs, XT *x, XT *__restrict__ aux, const double *__restrict__ dotv,
+    double *__restrict__ partials, DevScalars *sc, const int *stop, int defer, int coherent) {
   if (*stop) return;
   const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int wave =  // wave-uniform: the list comes through the scalar cache
+      __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
   int *err = &sc->err;
   double dacc = 0.0;
   __shared__ XT sbuf[4][64 * kStream];  // one stream-task product buffer per wave
@@ -278,55 +311,53 @@ __global__ __launch_bounds__(256) void k_sptrsv(
   // metadata of task k+1 are loaded before task k runs, so a task starts
   // with its rows, entry ranges and pivots already in registers.
   int k = wave_ptr[wave];
-  int n_info = 0, n_s0 = 0, n_row = 0, n_e0 = 0, n_e1 = 0;
-  VT n_dg = 1;
+  SweepTask nt = {0, 0, -1, 0};
+  RowMeta<VT> nm;
   auto fetch = [&](int kk) {
-    n_s0 = wt_s0[kk];
-    n_info = wt_info[kk];
-    if (((n_info >> kTaskInfoShift) & 15) != kTaskFlat &&
-        lane < (n_info & ((1 << kTaskInfoShift) - 1))) {
-      n_row = ld_stream(slot_row + n_s0 + lane);
-      n_e0 = ld_stream(rp + n_s0 + lane);
-      n_e1 = ld_stream(rp + n_s0 + lane + 1);
-      n_dg = ld_stream(diag + n_s0 + lane);
+    nt = wt[kk];
+    if (((nt.info >> kTaskInfoShift) & 15) != kTaskFlat &&
+        lane < (nt.info & ((1 << kTaskInfoShift) - 1))) {
+      const int *rq = (nt.info & kTaskMerged) ? mrp : rp;
+      nm.row = ld_stream(slot_row + nt.s0 + lane);
+      nm.e0 = ld_stream(rq + nt.s0 + lane);
+      nm.e1 = ld_stream(rq + nt.s0 + lane + 1);
+      nm.dg = ld_stream(diag + nt.s0 + lane);
     }
   };
   if (k < k1) fetch(k);
   for (; k < k1; k++) {
-    const int info = n_info, m_s0 = n_s0;
-    const int lg = (info >> kTaskInfoShift) & 15;
-    const int cnt = info & ((1 << kTaskInfoShift) - 1);  // <= 64 slots (flat: 64 kFlatPerLane)
-    const int px = info >> kTaskProxyShift;  // lane tasks' proxy (row_dot)
-    const int m_row = n_row, m_e0 = n_e0, m_e1 = n_e1;
-    const VT m_dg = n_dg;
+    const SweepTask t = nt;
+    const RowMeta<VT> m = nm;
+    const int lg = (t.info >> kTaskInfoShift) & 15;
+    const int cnt = t.info & ((1 << kTaskInfoShift) - 1);  // <= 64 slots (flat: 64 kFlatPerLane)
+    const bool merged = (t.info & kTaskMerged) != 0;
     if (!checked && lg != kTaskFlat) {  // the first task that may wait
       checked = true;
       if (!wave_resident(&sc->arrive, arrivals, err)) break;
     }
     if (k + 1 < k1) fetch(k + 1);
-#define RCHOL_SWEEP_TASK(LL)                                                                  \
-  sweep_task<VT, XT, BT, LL, FUSE>(cnt, m_row, m_e0, m_e1, m_dg, ci, cv, rhs, x, aux, dotv, err, \
-                                   coherent, dacc, px)
+#define RCHOL_SWEEP_LANES(LL)                                                                   \
+  sweep_lanes<VT, XT, BT, LL, FUSE>(cnt, m, merged ? mci : ci, merged ? mcv : cv, rhs, x, aux, \
+                                    dotv, err, coherent, dacc, merged, t.px)
     switch (lg) {
       case kTaskFlat:  // forward sweeps only (FUSE 0 / 1): keeps the r.z kernel's registers
         if constexpr (FUSE != 2)
-          sweep_flat<VT, XT, BT, FUSE>(m_s0, cnt, slot_row, diag, rhs, x, aux, dotv, dacc);
+          sweep_flat<VT, XT, BT, FUSE>(t.s0, cnt, slot_row, diag, rhs, x, aux, dotv, dacc);
         else
           atomicOr(err, 2);  // not in a backward schedule
         break;
       case kTaskStream:
-        sweep_stream<VT, XT, BT, FUSE>(cnt, m_row, m_e0, m_e1, m_dg, ci, cv, rhs, x, aux, dotv, err,
-                                       coherent, dacc, buf);
+        sweep_stream<VT, XT, BT, FUSE>(cnt, m, ci, cv, rhs, x, aux, dotv, err, coherent, dacc, buf);
         break;
-      case 0: RCHOL_SWEEP_TASK(1); break;
-      case 1: RCHOL_SWEEP_TASK(2); break;
-      case 2: RCHOL_SWEEP_TASK(4); break;
-      case 3: RCHOL_SWEEP_TASK(8); break;
-      case 4: RCHOL_SWEEP_TASK(16); break;
-      case 5: RCHOL_SWEEP_TASK(32); break;
-      default: RCHOL_SWEEP_TASK(64); break;
+      case 0: RCHOL_SWEEP_LANES(1); break;
+      case 1: RCHOL_SWEEP_LANES(2); break;
+      case 2: RCHOL_SWEEP_LANES(4); break;
+      case 3: RCHOL_SWEEP_LANES(8); break;
+      case 4: RCHOL_SWEEP_LANES(16); break;
+      case 5: RCHOL_SWEEP_LANES(32); break;
+      default: RCHOL_SWEEP_LANES(64); break;
     }
-#undef RCHOL_SWEEP_TASK
+#undef RCHOL_SWEEP_LANES
   }
   if (FUSE == 2) {
     double v[1] = {dacc}, tot[1];
@@ -342,6 +373,31 @@ __global__ __launch_bounds__(256) void k_sptrsv(
       }
     }
   }
+}
+
+// Sum of val[e] * x[ci[e]] over the entries [e0, e1) of one row by L lanes,
+// every input complete: rounds of kGather entries per lane from the row's
+// end.
+template <typename VT, typename XT, int L>
+__device__ __forceinline__ XT serial_dot(int e0, int e1, int sub, const int *__restrict__ ci,
+                                         const VT *__restrict__ cv, const XT *x) {
+  XT acc = 0;
+  for (int c = e1 - 1 - sub; c >= e0; c -= kGather * L) {
+    int j[kGather];
+    VT v[kGather];
+    XT xv[kGather];
+#pragma unroll
+    for (int u = 0; u < kGather; u++) {
+      const int e = c - u * L;
+      j[u] = e >= e0 ? ld_stream(ci + e) : -1;
+      v[u] = e >= e0 ? ld_stream(cv + e) : VT(0);
+    }
+#pragma unroll
+    for (int u = 0; u < kGather; u++) xv[u] = j[u] < 0 ? XT(0) : x[j[u]];
+#pragma unroll
+    for (int u = 0; u < kGather; u++) acc += (XT)v[u] * xv[u];
+  }
+  return acc;
 }
 
 // Rows [s0, s1) of one level in a 1024-thread workgroup, row groups of L
@@ -366,7 +422,7 @@ __device__ __forceinline__ void serial_level(int s0, int s1, const int *__restri
       e0 = rp[s];
       e1 = rp[s + 1];
     }
-    XT acc = row_dot<VT, XT, L, false>(e0, e1, sub, ci, cv, x, nullptr, 0);
+    XT acc = serial_dot<VT, XT, L>(e0, e1, sub, ci, cv, x);
     acc = group_sum<L>(acc);
     if (live && sub == 0) {
       const XT v = ((XT)rhs[row] - acc) / (XT)diag[s];

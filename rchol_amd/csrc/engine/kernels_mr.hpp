@@ -125,10 +125,7 @@ __device__ __forceinline__ XT row_dot_mr(int e0, int e1, int sub, int c,
     }
 #pragma unroll
     for (int u = 0; u < kGather; u++) xv[u] = j[u] < 0 ? XT(0) : x[(size_t)j[u] * K + c];
-    bool pend = false;
-#pragma unroll
-    for (int u = 0; u < kGather; u++) pend |= Sent<XT>::is(xv[u]);
-    if (__ballot(pend)) await_batch<XT, kGather>(x, j, xv, err, K, c);
+    if (pending_lanes(j, xv)) await_batch<XT, kGather>(x, j, xv, err, K, c);
 #pragma unroll
     for (int u = 0; u < kGather; u++) acc += (XT)v[u] * xv[u];
   }
@@ -169,8 +166,8 @@ __device__ __forceinline__ void sweep_task_mr(int cnt, int m_row, int m_e0, int 
 
 template <typename VT, typename XT, typename BT, int K, int FUSE>
 __global__ __launch_bounds__(256) void k_sptrsv_mr(
-    const int *__restrict__ wave_ptr, const int *__restrict__ wt_s0,
-    const int *__restrict__ wt_info, const int *__restrict__ slot_row,
+    const int *__restrict__ wave_ptr, const SweepTask *__restrict__ wt,
+    const int *__restrict__ slot_row,
     const int *__restrict__ rp, const int *__restrict__ ci, const VT *__restrict__ cv,
     const VT *__restrict__ diag, const BT *__restrict__ rhs, XT *x, XT *__restrict__ aux,
     const double *__restrict__ dotv, double *__restrict__ partials, BatchScalars *bs,
@@ -186,8 +183,8 @@ __global__ __launch_bounds__(256) void k_sptrsv_mr(
   int n_info = 0, n_row = 0, n_e0 = 0, n_e1 = 0;
   VT n_dg = 1;
   auto fetch = [&](int kk) {
-    const int s = wt_s0[kk];
-    n_info = wt_info[kk];
+    const int s = wt[kk].s0;
+    n_info = wt[kk].info;
     if (lane < (n_info & ((1 << kTaskInfoShift) - 1))) {
       n_row = ld_stream(slot_row + s + lane);
       n_e0 = ld_stream(rp + s + lane);

@@ -26,6 +26,7 @@ OPT_TASK_WAVES = 8
 OPT_STRICT_SYNC = 9
 OPT_CHUNKED = 10
 OPT_WAIT_TICKS = 11
+OPT_MERGE = 12
 
 
 class Stats(ctypes.Structure):
@@ -396,6 +397,30 @@ def chunk_apply_host(G, r, max_rows=65535):
     return z, cnt.tolist(), nrd.value, est
 
 
+def merge_apply_host(G, r):
+    """The merged-level plan of the persistent sweeps for G, run on the host:
+    z = G^-T G^-1 r.  Returns (z, groups, entries of merged rows, estimates in
+    microseconds), the last three as [forward, backward]."""
+    if isinstance(G, tuple):
+        cp, ri, gv = G
+    else:
+        cp, ri, gv = stored_from_lower(G)
+    cp, pcp = _u64(cp)
+    ri, pri = _u64(ri)
+    gv, pgv = _f64(gv)
+    r, pr = _f64(r)
+    z = np.empty_like(r)
+    groups = np.zeros(2, dtype=np.int32)
+    ents = (ctypes.c_longlong * 2)()
+    est = np.zeros(2)
+    lib = _lib.engine()
+    _lib.check(lib.rchol_amd_merge_apply_host(cp.size - 1, pcp, pri, pgv, pr,
+                                              z.ctypes.data_as(_lib.f64p),
+                                              groups.ctypes.data_as(_lib.i32p), ents,
+                                              est.ctypes.data_as(_lib.f64p)))
+    return z, groups.tolist(), list(ents), est.tolist()
+
+
 def pcg(A, b, epsilon, maxitr, G, Gt=None):
     """Drop-in for python/rchol/util.py:32-61: pcg(A, b, epsilon, maxitr, G, Gt).
 
@@ -405,5 +430,7 @@ def pcg(A, b, epsilon, maxitr, G, Gt=None):
     ||A x - b|| / ||b|| (util.py:56).  The preconditioner applied is
     G^-T G^-1 as in c++/util/pcg.cpp:141-159.
     """
-    with Solver(A, G) as s:
+    with Solver(A) as s:
+        s.set_option(OPT_MERGE, 0)  # one solve does not earn the merged levels back
+        s.upload_G(G)
         return s.pcg(b, epsilon, maxitr)

@@ -71,10 +71,9 @@ template <> struct Sent<float> {
   }
 };
 
-// Loads of data that a kernel reads exactly once (matrix indices and
-// values, per-slot metadata, the right-hand side): non-temporal, so that
-// the L2 keeps the gathered vector lines that neighbouring rows reuse
-// instead of filling with the streamed matrix.
+// Loads of data that a kernel reads exactly once, non-temporal, so that the
+// L2 keeps the gathered vector lines that neighbouring rows reuse instead of
+// filling with the streamed matrix (K-column kernels, chunked sweeps).
 #ifndef RCHOL_AMD_NT
 #define RCHOL_AMD_NT 1
 #endif
@@ -85,6 +84,15 @@ __device__ __forceinline__ T ld_stream(const T *p) {
 #else
   return *p;
 #endif
+}
+// The same as a choice of the kernel.  The single-column sweeps load plainly
+// at every size (both sweeps, non-temporal -> plain: 97x61x83 FP32 0.33 ->
+// 0.31 ms, 128^3 FP32 0.73 -> 0.70 ms, 256^3 2.60 -> 2.55 ms: their matrices
+// come back from the Infinity Cache as far as they fit it).
+template <bool NT, typename T>
+__device__ __forceinline__ T ld_once(const T *p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  return *p;
 }
 
 // Bound on one dependency wait, in wall-clock ticks (the constant-rate

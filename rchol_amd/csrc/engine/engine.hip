@@ -532,6 +532,11 @@ struct rchol_amd_ctx {
     if (g > 8) g = (g + 7) / 8 * 8;  // whole XCD rounds for the row walk of the stream form
     return (int)g;
   }
+  // A larger than half the Infinity Cache streams past the caches in the SpMV,
+  // a smaller one is left in them for the next iteration (stream form, plain
+  // / non-temporal: 48 ... 100^3 and 2D stacks 5 to 10% faster plain, 97x61x83
+  // 26.4 / 28.7 us; 128^3 77 / 75 us, 160^3 139 / 132 us)
+  bool spmv_nt() const { return nnzA * 12 > (128u << 20); }
   int ensure_work();
   int size_trsv_grid();
   int launch_iteration(int parity, int slot);
@@ -640,9 +645,9 @@ void launch_spmv_p(rchol_amd_ctx *c, const ZT *z, const double *p_old, double *p
     case 0:
       hipLaunchKernelGGL((k_p_update<ZT>), dim3(c->vec_grid()), dim3(kBlock), 0, c->stream,
                          (int)c->n, z, p_old, p_new, c->sc);
-      hipLaunchKernelGGL(k_spmv_p_s, dim3(c->spmv_grid()), dim3(kBlock), 0, c->stream, (int)c->n,
-                         c->arp.p, c->aci.p, c->av.p, (const double *)p_new, c->q.p, c->r.p,
-                         c->partials.p, c->sc);
+      hipLaunchKernelGGL(c->spmv_nt() ? k_spmv_p_s<true> : k_spmv_p_s<false>, dim3(c->spmv_grid()),
+                         dim3(kBlock), 0, c->stream, (int)c->n, c->arp.p, c->aci.p, c->av.p,
+                         (const double *)p_new, c->q.p, c->r.p, c->partials.p, c->sc);
       break;
     case 4: launch_spmv_p_t<ZT, 4>(c, z, p_old, p_new); break;
     case 16: launch_spmv_p_t<ZT, 16>(c, z, p_old, p_new); break;
@@ -681,8 +686,9 @@ void launch_resid_replace(rchol_amd_ctx *c) {
 void launch_spmv_res(rchol_amd_ctx *c, const double *x, const double *b, double *y) {
   switch (c->spmv_lanes) {
     case 0:
-      hipLaunchKernelGGL(k_spmv_res_s, dim3(c->spmv_grid()), dim3(kBlock), 0, c->stream, (int)c->n,
-                         c->arp.p, c->aci.p, c->av.p, x, b, y, c->partials.p, c->sc);
+      hipLaunchKernelGGL(c->spmv_nt() ? k_spmv_res_s<true> : k_spmv_res_s<false>,
+                         dim3(c->spmv_grid()), dim3(kBlock), 0, c->stream, (int)c->n, c->arp.p,
+                         c->aci.p, c->av.p, x, b, y, c->partials.p, c->sc);
       break;
     case 4: launch_spmv_res_t<4>(c, x, b, y); break;
     case 16: launch_spmv_res_t<16>(c, x, b, y); break;
@@ -716,6 +722,20 @@ static int trsv_occupancy() {
   return std::min(a, std::min(b, c));
 }
 
+// Workgroups of the persistent sweeps for a cut of T tasks, below the
+// resident capacity: waves that are far ahead of their inputs only poll, so
+// few tasks want few waves -- half a wave per task up to 768 waves, then
+// 12 sqrt(T).  Both sweeps, one wave per task (up to the capacity) -> this:
+// 20^3 (1.3 k tasks) 49 -> 43 us, 32^3 (3 k) 86 -> 76, 48^3 FP32 (7 k) 166 ->
+// 148, 64^3 FP32 (13 k) 238 -> 220, 97x61x83 FP32 (21 k) 306 -> 291; from
+// 70 k tasks on every resident wave helps (128^3 FP32 at two thirds: +1%).
+static size_t sweep_blocks(size_t tasks) {
+  const size_t waves = std::max<size_t>(std::min<size_t>(tasks / 2, 768),
+                                        (size_t)(12.0 * std::sqrt((double)tasks)));
+  size_t b = std::min((waves + 3) / 4, (tasks + 3) / 4);
+  return b > 8 ? (b + 7) / 8 * 8 : b;  // whole XCD rounds
+}
+
 // Grid of the persistent sweeps and the task cut that goes with it: the
 // resident capacity fixes how finely narrow levels are split.
 int rchol_amd_ctx::size_trsv_grid() {
@@ -736,7 +756,7 @@ int rchol_amd_ctx::size_trsv_grid() {
     cut_tasks(*sw[k], h[k], t[k], lmin_lg, plan_waves, k == 0, serial_width == 0, tc[k]);
     max_tasks = std::max(max_tasks, tc[k].s0.size());
   }
-  trsv_grid = (int)std::max<size_t>(1, std::min<size_t>(cap_blocks, (max_tasks + 3) / 4));
+  trsv_grid = (int)std::max<size_t>(1, std::min<size_t>(cap_blocks, sweep_blocks(max_tasks)));
   // the residency check counts arrivals in whole grids: restart the count
   HIP_TRY(hipMemset(&sc->arrive, 0, sizeof(sc->arrive)));
   for (int k = 0; k < 2; k++) HIP_TRY(upload_schedule(*sw[k], h[k], t[k], lmin_lg, tc[k], trsv_grid));
@@ -1251,7 +1271,8 @@ void launch_spmv_p_seg_t(rchol_amd_ctx *c, SegLayout lay, const void *z, bool z3
     else
       hipLaunchKernelGGL((k_p_update_seg<double>), dim3(c->segs.nblocks), dim3(kBlock), 0,
                          c->stream, lay, (const double *)z, p_old, p_new, c->segs.ss);
-    hipLaunchKernelGGL(k_spmv_p_seg_s, dim3(c->segs.nblocks), dim3(kBlock), 0, c->stream, lay,
+    hipLaunchKernelGGL(c->spmv_nt() ? k_spmv_p_seg_s<true> : k_spmv_p_seg_s<false>,
+                       dim3(c->segs.nblocks), dim3(kBlock), 0, c->stream, lay,
                        c->arp.p, c->aci.p, c->av.p, (const double *)p_new, c->q.p,
                        (const double *)c->r.p, c->partials.p, c->segs.ss);
     return;
@@ -1387,7 +1408,7 @@ int rchol_amd_ctx::pcg_segments(const double *d_b, double tol, int maxit, double
   if (hsc->err)
     return stall(hsc->err);
   switch (spmv_lanes) {
-    case 0: hipLaunchKernelGGL(k_spmv_res_seg_s, dim3(segs.nblocks), dim3(kBlock), 0, stream, lay, arp.p, aci.p, av.p, (const double *)x.p, d_b, tmp64a.p, partials.p, segs.ss); break;
+    case 0: hipLaunchKernelGGL(spmv_nt() ? k_spmv_res_seg_s<true> : k_spmv_res_seg_s<false>, dim3(segs.nblocks), dim3(kBlock), 0, stream, lay, arp.p, aci.p, av.p, (const double *)x.p, d_b, tmp64a.p, partials.p, segs.ss); break;
     case 4: hipLaunchKernelGGL((k_spmv_res_seg<4>), dim3(segs.nblocks), dim3(kBlock), 0, stream, lay, arp.p, aci.p, av.p, (const double *)x.p, d_b, tmp64a.p, partials.p, segs.ss); break;
     case 16: hipLaunchKernelGGL((k_spmv_res_seg<16>), dim3(segs.nblocks), dim3(kBlock), 0, stream, lay, arp.p, aci.p, av.p, (const double *)x.p, d_b, tmp64a.p, partials.p, segs.ss); break;
     case 32: hipLaunchKernelGGL((k_spmv_res_seg<32>), dim3(segs.nblocks), dim3(kBlock), 0, stream, lay, arp.p, aci.p, av.p, (const double *)x.p, d_b, tmp64a.p, partials.p, segs.ss); break;

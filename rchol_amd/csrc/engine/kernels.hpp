@@ -89,8 +89,8 @@ __device__ __forceinline__ XT row_dot(int e0, int e1, int sub, const int *__rest
 #pragma unroll
     for (int u = 0; u < kGather; u++) {
       const int e = c - u * L;
-      j[u] = e >= e0 ? ld_stream(ci + e) : -1;
-      v[u] = e >= e0 ? ld_stream(cv + e) : VT(0);
+      j[u] = e >= e0 ? ci[e] : -1;
+      v[u] = e >= e0 ? cv[e] : VT(0);
     }
     const bool proxy = RCHOL_AMD_PROXY && px >= 0 && r == 0;
     if (proxy) await_value(x + px, err);
@@ -146,7 +146,7 @@ __device__ __forceinline__ void sweep_lanes(int cnt, const RowMeta<VT> &m,
   if (!live) e1 = e0;
   const bool writes = live && sub == 0;
   // before the waits: what the epilogue needs besides the sum
-  const BT b = writes ? ld_stream(rhs + row) : (BT)0;
+  const BT b = writes ? rhs[row] : (BT)0;
   const double dv = FUSE == 2 && writes ? dotv[row] : 0.0;
   XT acc = row_dot<VT, XT, BT, L>(e0, e1, sub, ci, cv, x, rhs, err, coherent, merged, px);
   acc = group_sum<L>(acc);
@@ -210,7 +210,7 @@ __device__ __forceinline__ void sweep_stream(int cnt, const RowMeta<VT> &m,
   const int m_row = m.row, m_e0 = m.e0, m_e1 = m.e1;
   const VT m_dg = m.dg;
   const int E0 = __shfl(m_e0, 0, 64), E1 = __shfl(m_e1, cnt - 1, 64);
-  const BT b = live ? ld_stream(rhs + m_row) : (BT)0;
+  const BT b = live ? rhs[m_row] : (BT)0;
   const double dv = FUSE == 2 && live ? dotv[m_row] : 0.0;
   XT acc = 0;
   for (int c = E0; c < E1; c += 64 * kStream) {
@@ -220,8 +220,8 @@ __device__ __forceinline__ void sweep_stream(int cnt, const RowMeta<VT> &m,
 #pragma unroll
     for (int u = 0; u < kStream; u++) {
       const int e = c + u * 64 + lane;
-      j[u] = e < E1 ? ld_stream(ci + e) : -1;
-      v[u] = e < E1 ? ld_stream(cv + e) : VT(0);
+      j[u] = e < E1 ? ci[e] : -1;
+      v[u] = e < E1 ? cv[e] : VT(0);
     }
 #pragma unroll
     for (int u = 0; u < kStream; u++) {
@@ -274,11 +274,11 @@ __device__ __forceinline__ void sweep_flat(int s0, int cnt, const int *__restric
 #pragma unroll
   for (int u = 0; u < kFlatPerLane; u++) {
     const int t = u * 64 + lane;
-    row[u] = t < cnt ? ld_stream(slot_row + s0 + t) : -1;
-    dg[u] = t < cnt ? ld_stream(diag + s0 + t) : VT(1);
+    row[u] = t < cnt ? slot_row[s0 + t] : -1;
+    dg[u] = t < cnt ? diag[s0 + t] : VT(1);
   }
 #pragma unroll
-  for (int u = 0; u < kFlatPerLane; u++) b[u] = row[u] >= 0 ? ld_stream(rhs + row[u]) : (BT)0;
+  for (int u = 0; u < kFlatPerLane; u++) b[u] = row[u] >= 0 ? rhs[row[u]] : (BT)0;
 #pragma unroll
   for (int u = 0; u < kFlatPerLane; u++) {
     if (row[u] < 0) continue;
@@ -318,10 +318,10 @@ __global__ __launch_bounds__(256) void k_sptrsv(
     if (((nt.info >> kTaskInfoShift) & 15) != kTaskFlat &&
         lane < (nt.info & ((1 << kTaskInfoShift) - 1))) {
       const int *rq = (nt.info & kTaskMerged) ? mrp : rp;
-      nm.row = ld_stream(slot_row + nt.s0 + lane);
-      nm.e0 = ld_stream(rq + nt.s0 + lane);
-      nm.e1 = ld_stream(rq + nt.s0 + lane + 1);
-      nm.dg = ld_stream(diag + nt.s0 + lane);
+      nm.row = slot_row[nt.s0 + lane];
+      nm.e0 = rq[nt.s0 + lane];
+      nm.e1 = rq[nt.s0 + lane + 1];
+      nm.dg = diag[nt.s0 + lane];
     }
   };
   if (k < k1) fetch(k);
@@ -340,8 +340,9 @@ __global__ __launch_bounds__(256) void k_sptrsv(
   sweep_lanes<VT, XT, BT, LL, FUSE>(cnt, m, merged ? mci : ci, merged ? mcv : cv, rhs, x, aux, \
                                     dotv, err, coherent, dacc, merged, t.px)
     switch (lg) {
-      case kTaskFlat:  // forward sweeps only (FUSE 0 / 1): keeps the r.z kernel's registers
-        if constexpr (FUSE != 2)
+      case kTaskFlat:  // forward sweeps only: its registers weigh on every task (256^3 FP32,
+                       // backward sweep of one application: 1.43 ms with it, 1.11 ms without)
+        if constexpr (FUSE == 1)
           sweep_flat<VT, XT, BT, FUSE>(t.s0, cnt, slot_row, diag, rhs, x, aux, dotv, dacc);
         else
           atomicOr(err, 2);  // not in a backward schedule
@@ -742,14 +743,14 @@ __device__ __forceinline__ RowWalk xcd_rows(int n) {
 // sum_e av[e] * g(ci[e]) over the entries of row r0 + lane (lanes whose row
 // is >= n, the end of the walk, return 0).  buf: this wave's
 // 64 * kSpmvStream doubles of LDS.
-template <typename G>
+template <bool NT, typename G>
 __device__ __forceinline__ double stream_rows(int r0, int n, const int *__restrict__ rp,
                                               const int *__restrict__ ci,
                                               const double *__restrict__ av, G g, double *buf) {
   const int lane = threadIdx.x & 63;
   const int row = r0 + lane;
   const bool live = row < n;
-  const int e0 = live ? ld_stream(rp + row) : 0, e1 = live ? ld_stream(rp + row + 1) : 0;
+  const int e0 = live ? ld_once<NT>(rp + row) : 0, e1 = live ? ld_once<NT>(rp + row + 1) : 0;
   const int last = min(64, n - r0) - 1;
   const int E0 = __shfl(e0, 0, 64), E1 = __shfl(e1, last, 64);
   double acc = 0.0;
@@ -759,8 +760,8 @@ __device__ __forceinline__ double stream_rows(int r0, int n, const int *__restri
 #pragma unroll
     for (int u = 0; u < kSpmvStream; u++) {
       const int e = c + u * 64 + lane;
-      j[u] = e < E1 ? ld_stream(ci + e) : -1;
-      a[u] = e < E1 ? ld_stream(av + e) : 0.0;
+      j[u] = e < E1 ? ld_once<NT>(ci + e) : -1;
+      a[u] = e < E1 ? ld_once<NT>(av + e) : 0.0;
     }
 #pragma unroll
     for (int u = 0; u < kSpmvStream; u++) pv[u] = j[u] >= 0 ? g(j[u]) : 0.0;
@@ -798,6 +799,7 @@ __global__ __launch_bounds__(256) void k_p_update(int n, const ZT *__restrict__ 
 
 // k_spmv_p in stream form, after k_p_update: q = A p', p'.r, p'.q and alpha
 // (same results up to the order of each row sum).
+template <bool NT>
 __global__ __launch_bounds__(256) void k_spmv_p_s(int n, const int *__restrict__ rp,
                                                   const int *__restrict__ ci,
                                                   const double *__restrict__ av,
@@ -818,7 +820,7 @@ __global__ __launch_bounds__(256) void k_spmv_p_s(int n, const int *__restrict__
       pi = p[row];
       ri = r[row];
     }
-    const double acc = stream_rows(r0, rw.hi, rp, ci, av, [&](int j) { return p[j]; }, buf);
+    const double acc = stream_rows<NT>(r0, rw.hi, rp, ci, av, [&](int j) { return p[j]; }, buf);
     if (row < rw.hi) {
       q[row] = acc;
       apr += pi * ri;
@@ -850,7 +852,7 @@ __global__ __launch_bounds__(256) void k_resid_replace_s(int n, const int *__res
   for (int r0 = rw.first; r0 < rw.hi; r0 += rw.step) {
     const int row = r0 + lane;
     const double bi = row < rw.hi ? bvec[row] : 0.0;
-    const double acc = stream_rows(r0, rw.hi, rp, ci, av, [&](int j) { return x[j]; }, buf);
+    const double acc = stream_rows<true>(r0, rw.hi, rp, ci, av, [&](int j) { return x[j]; }, buf);
     if (row < rw.hi) {
       const double ri = bi - acc;
       r[row] = ri;
@@ -865,6 +867,7 @@ __global__ __launch_bounds__(256) void k_resid_replace_s(int n, const int *__res
 }
 
 // k_spmv_res in stream form.
+template <bool NT>
 __global__ __launch_bounds__(256) void k_spmv_res_s(int n, const int *__restrict__ rp,
                                                     const int *__restrict__ ci,
                                                     const double *__restrict__ av,
@@ -880,7 +883,7 @@ __global__ __launch_bounds__(256) void k_spmv_res_s(int n, const int *__restrict
   for (int r0 = rw.first; r0 < rw.hi; r0 += rw.step) {
     const int row = r0 + lane;
     const double bi = (bvec && row < rw.hi) ? bvec[row] : 0.0;
-    double acc = stream_rows(r0, rw.hi, rp, ci, av, [&](int j) { return x[j]; }, buf);
+    double acc = stream_rows<NT>(r0, rw.hi, rp, ci, av, [&](int j) { return x[j]; }, buf);
     if (row < rw.hi) {
       acc -= bi;
       y[row] = acc;

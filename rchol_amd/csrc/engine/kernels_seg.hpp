@@ -213,6 +213,7 @@ __global__ __launch_bounds__(256) void k_p_update_seg(SegLayout lay, const ZT *_
 // (stream_rows), gathering p'.
 // Occupancy 8 (<= 64 VGPRs): the grid fills 8 workgroups per CU, and at 7
 // resident the eighth would run as a second wave of workgroups.
+template <bool NT>
 __global__ __launch_bounds__(256, 8) void k_spmv_p_seg_s(SegLayout lay, const int *__restrict__ rp,
                                                       const int *__restrict__ ci,
                                                       const double *__restrict__ av,
@@ -234,7 +235,7 @@ __global__ __launch_bounds__(256, 8) void k_spmv_p_seg_s(SegLayout lay, const in
       pi = p[row];
       ri = r[row];
     }
-    const double acc = stream_rows(r0, hi, rp, ci, av, [&](int j) { return p[j]; }, buf);
+    const double acc = stream_rows<NT>(r0, hi, rp, ci, av, [&](int j) { return p[j]; }, buf);
     if (row < hi) {
       q[row] = acc;
       apr += pi * ri;
@@ -319,6 +320,7 @@ __global__ __launch_bounds__(256) void k_spmv_res_seg(SegLayout lay, const int *
 }
 
 // k_spmv_res_seg in stream form.
+template <bool NT>
 __global__ __launch_bounds__(256) void k_spmv_res_seg_s(SegLayout lay, const int *__restrict__ rp,
                                                         const int *__restrict__ ci,
                                                         const double *__restrict__ av,
@@ -335,7 +337,7 @@ __global__ __launch_bounds__(256) void k_spmv_res_seg_s(SegLayout lay, const int
   for (int r0 = lay.r0[blockIdx.x] + wv * 64; r0 < hi; r0 += nwv * 64) {
     const int row = r0 + lane;
     const double bi = row < hi ? bvec[row] : 0.0;
-    double acc = stream_rows(r0, hi, rp, ci, av, [&](int j) { return x[j]; }, buf);
+    double acc = stream_rows<NT>(r0, hi, rp, ci, av, [&](int j) { return x[j]; }, buf);
     if (row < hi) {
       acc -= bi;
       y[row] = acc;

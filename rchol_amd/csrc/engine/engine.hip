@@ -83,13 +83,6 @@ constexpr int kTaskRows = 64;     // slots per triangular-sweep task
 #define RCHOL_AMD_SPMV_PER_CU 2
 #endif
 constexpr int kSpmvBlocksPerCu = RCHOL_AMD_SPMV_PER_CU;
-// The K-column SpMV gathers K values per entry and needs more rows in flight
-// (K = 32 at 256^3, ms per SpMV: 4 per CU 12.7, 5 11.5, 6 10.9, 7 11.1,
-// 8 12.1).
-#ifndef RCHOL_AMD_SPMV_MR_PER_CU
-#define RCHOL_AMD_SPMV_MR_PER_CU 6
-#endif
-constexpr int kSpmvMrBlocksPerCu = RCHOL_AMD_SPMV_MR_PER_CU;
 #ifndef RCHOL_AMD_VEC_PER_CU
 #define RCHOL_AMD_VEC_PER_CU 4
 #endif
@@ -305,20 +298,21 @@ void cut_tasks(const Sweep &sw, int h, int t, int lmin_lg, long long nwaves, boo
 // entry-lane width Le = 2^lg <= 64/K (a row takes K * Le lanes) that covers
 // the longest of the run's rows in one round of kGather gathers, R = 64/(K Le)
 // rows per pass; narrow levels get one-pass tasks, wide ones as many passes
-// (at most 64 slots) as it takes to need about one task per wave.
-void cut_tasks_mr(const std::vector<int> &lp, const std::vector<int> &rp, int nlevels, int K,
-                  long long nwaves, TaskCut &tc) {
+// (at most 64 slots) as it takes to need about one task per wave.  With merge,
+// a group of merged levels is one level (as in cut_tasks).
+void cut_tasks_mr(const Sweep &sw, int K, long long nwaves, bool merge, TaskCut &tc) {
+  const std::vector<int> &lp = sw.level_ptr_h;
   tc.s0.clear();
   tc.info.clear();
   tc.px.clear();
   tc.level.clear();
   int maxlg = 0;
   while ((K << (maxlg + 1)) <= 64) maxlg++;
-  for (int l = 0; l < nlevels; l++) {
-    const int s_end = lp[l + 1];
-    const long long rows = s_end - lp[l];
-    for (int s = lp[l]; s < s_end;) {
-      int lg = std::min(lane_lg(rp[s + 1] - rp[s], 0), maxlg), take = 0;
+  auto cut = [&](int s, int s_end, int l, const int *rp, int flag) {
+    const long long rows = s_end - s;
+    auto lg_of = [&](int k) { return std::min(lane_lg(rp[k + 1] - rp[k], 0), maxlg); };
+    while (s < s_end) {
+      int lg = lg_of(s), take = 0;
       for (;;) {
         const int R = 64 / (K << lg);
         const long long one_pass = (rows + R - 1) / R;
@@ -326,17 +320,33 @@ void cut_tasks_mr(const std::vector<int> &lp, const std::vector<int> &rp, int nl
             (int)std::min<long long>(64 / R, std::max<long long>(1, (one_pass + nwaves - 1) / nwaves));
         take = std::min(s_end - s, passes * R);
         int need = lg;
-        for (int k = 0; k < take; k++)
-          need = std::max(need, std::min(lane_lg(rp[s + k + 1] - rp[s + k], 0), maxlg));
+        for (int k = 0; k < take; k++) need = std::max(need, lg_of(s + k));
         if (need == lg) break;
         lg = need;
       }
       tc.s0.push_back(s);
-      tc.info.push_back(take | (lg << kTaskInfoShift));
+      tc.info.push_back(take | (lg << kTaskInfoShift) | flag);
       tc.px.push_back(-1);
       tc.level.push_back(l);
       s += take;
     }
+  };
+  const int *rp = sw.rp_h.data();
+  if (!merge || sw.m1 == sw.m0) {
+    for (int l = 0; l < sw.nlevels; l++) cut(lp[l], lp[l + 1], l, rp, 0);
+    return;
+  }
+  const int *mrp = sw.mrp_h.data() - sw.m0;
+  for (size_t g = 0; g + 1 < sw.gptr_h.size(); g++) {
+    const int a = sw.gptr_h[g], b = sw.gptr_h[g + 1];
+    // merged rows fill their lanes: those of a group have to fit the waves
+    const bool fits = (long long)(lp[b] - lp[a]) * (K << maxlg) <= 64 * nwaves;
+    if (b - a == 1 || !fits) {
+      for (int l = a; l < b; l++) cut(lp[l], lp[l + 1], l, rp, 0);
+      continue;
+    }
+    cut(lp[a], lp[a + 1], a, rp, 0);
+    cut(lp[a + 1], lp[b], a, mrp, kTaskMerged);
   }
 }
 
@@ -536,6 +546,16 @@ struct rchol_amd_ctx {
   // a smaller one is left in them for the next iteration (stream form, plain
   // / non-temporal: 48 ... 100^3 and 2D stacks 5 to 10% faster plain, 97x61x83
   // 26.4 / 28.7 us; 128^3 77 / 75 us, 160^3 139 / 132 us)
+  // Grid of the K-column SpMV (kCols columns per lane): at least two row steps
+  // per wave, since every workgroup adds to the reduction that ends the kernel
+  // (24^3, K = 32: 40 us with one step, 28 with two, 29 with eight), whole XCD
+  // rounds for the row walk
+  int spmv_mr_grid(int K) const {
+    const size_t rows_per_block = 2 * (kBlock / 64) * (64 / (K / kCols));
+    size_t g = std::max<size_t>(1, std::min<size_t>((n + rows_per_block - 1) / rows_per_block,
+                                                    (size_t)ncu * kSpmvMrBlocksPerCu));
+    return (int)(g > 8 ? (g + 7) / 8 * 8 : g);
+  }
   bool spmv_nt() const { return nnzA * 12 > (128u << 20); }
   int ensure_work();
   int size_trsv_grid();
@@ -1012,10 +1032,10 @@ int rchol_amd_ctx::ensure_batch_schedule(int K, int per_cu) {
   Sweep *sw[2] = {&fwd, &bwd};
   size_t max_tasks = 0;
   for (int k = 0; k < 2; k++) {
-    cut_tasks_mr(sw[k]->level_ptr_h, sw[k]->rp_h, sw[k]->nlevels, K, plan_waves, tc[k]);
+    cut_tasks_mr(*sw[k], K, plan_waves, K <= kMergeCols, tc[k]);
     max_tasks = std::max(max_tasks, tc[k].s0.size());
   }
-  batch.grid = (int)std::max<size_t>(1, std::min<size_t>(cap_blocks, (max_tasks + 3) / 4));
+  batch.grid = (int)std::max<size_t>(1, std::min<size_t>(cap_blocks, sweep_blocks(max_tasks)));
   HIP_TRY(hipMemset(&batch.bs->arrive, 0, sizeof(batch.bs->arrive)));
   for (int k = 0; k < 2; k++) {
     std::vector<int> wp;
@@ -1036,28 +1056,31 @@ void rchol_amd_ctx::launch_sweeps_mr(const double *rhs, bool with_dot, const int
   const dim3 g(batch.grid), blk(kBlock);
   const int *wpf = batch.wave_ptr[0].p, *wpb = batch.wave_ptr[1].p;
   const SweepTask *wtf = batch.wt[0].p, *wtb = batch.wt[1].p;
+  // indexed by slot
+  const int *mrpf = fwd.mrp.p ? fwd.mrp.p - fwd.m0 : nullptr;
+  const int *mrpb = bwd.mrp.p ? bwd.mrp.p - bwd.m0 : nullptr;
   if (gprec == RCHOL_AMD_FP32) {
-    hipLaunchKernelGGL((k_sptrsv_mr<float, float, double, K, 1>), g, blk, 0, stream, wpf, wtf, fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv32.p, fwd.diag32.p, rhs,
+    hipLaunchKernelGGL((k_sptrsv_mr<float, float, double, K, 1>), g, blk, 0, stream, wpf, wtf, fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv32.p, mrpf, fwd.mci.p, fwd.mcv32.p, fwd.diag32.p, rhs,
                        batch.y32.p, batch.z32.p, nullptr, nullptr, batch.bs, stop);
     if (ev) (void)hipEventRecord(ev[1], stream);
     if (with_dot)
-      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 2>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, bwd.diag32.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 2>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, mrpb, bwd.mci.p, bwd.mcv32.p, bwd.diag32.p,
                          (const float *)batch.y32.p, batch.z32.p, (float *)nullptr,
                          (const double *)batch.r.p, batch.partials.p, batch.bs, stop);
     else
-      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 0>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, bwd.diag32.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 0>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, mrpb, bwd.mci.p, bwd.mcv32.p, bwd.diag32.p,
                          (const float *)batch.y32.p, batch.z32.p, (float *)nullptr, nullptr,
                          nullptr, batch.bs, stop);
   } else {
-    hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 1>), g, blk, 0, stream, wpf, wtf, fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv64.p, fwd.diag64.p, rhs,
+    hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 1>), g, blk, 0, stream, wpf, wtf, fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv64.p, mrpf, fwd.mci.p, fwd.mcv64.p, fwd.diag64.p, rhs,
                        batch.y64.p, batch.z64.p, nullptr, nullptr, batch.bs, stop);
     if (ev) (void)hipEventRecord(ev[1], stream);
     if (with_dot)
-      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 2>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, bwd.diag64.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 2>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, mrpb, bwd.mci.p, bwd.mcv64.p, bwd.diag64.p,
                          (const double *)batch.y64.p, batch.z64.p, (double *)nullptr,
                          (const double *)batch.r.p, batch.partials.p, batch.bs, stop);
     else
-      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 0>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, bwd.diag64.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 0>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, mrpb, bwd.mci.p, bwd.mcv64.p, bwd.diag64.p,
                          (const double *)batch.y64.p, batch.z64.p, (double *)nullptr, nullptr,
                          nullptr, batch.bs, stop);
   }
@@ -1071,24 +1094,26 @@ void rchol_amd_ctx::launch_iteration_mr(int parity, int slot) {
   hipEvent_t *ev = profile ? &pev[(size_t)slot * 5] : nullptr;
   if (ev) (void)hipEventRecord(ev[0], stream);
   launch_sweeps_mr<K>(batch.r.p, true, &batch.bs->all_done, ev);
-  const int rows_per_block = (kBlock / 64) * (64 / K);
-  int sg = (int)std::max<size_t>(
-      1, std::min<size_t>((n + rows_per_block - 1) / rows_per_block, (size_t)ncu * kSpmvMrBlocksPerCu));
-  if (sg > 8) sg = (sg + 7) / 8 * 8;  // whole XCD rounds for the row walk
-  const int vg = (int)std::max<size_t>(
-      1, std::min<size_t>((n * K + kBlock - 1) / kBlock, (size_t)ncu * kVecBlocksPerCu));
+  const int sg = spmv_mr_grid(K);
+  const size_t pairs = 2 * kBlock;  // two steps of a block: 24^3, K = 32: 28 us with one, 20 with two
+  const int vg = (int)std::max<size_t>(1, std::min<size_t>((n * (K / kCols) + pairs - 1) / pairs,
+                                                           (size_t)ncu * kVecBlocksPerCu));
   if (gprec == RCHOL_AMD_FP32) {
-    hipLaunchKernelGGL((k_spmv_p_mr<float, K>), dim3(sg), dim3(kBlock), 0, stream, (int)n,
-                       arp.p, aci.p, av.p, (const float *)batch.z32.p, (const double *)p_old,
-                       p_new, batch.q.p, (const double *)batch.r.p, batch.partials.p, batch.bs);
+    hipLaunchKernelGGL((k_p_update_mr<float, K>), dim3(vg), dim3(kBlock), 0, stream, (int)n,
+                       (const float *)batch.z32.p, (const double *)p_old, p_new, batch.bs);
+    hipLaunchKernelGGL((k_spmv_p_mr<K>), dim3(sg), dim3(kBlock), 0, stream, (int)n, arp.p, aci.p,
+                       av.p, (const double *)p_new, batch.q.p, (const double *)batch.r.p,
+                       batch.partials.p, batch.bs);
     if (ev) (void)hipEventRecord(ev[3], stream);
     hipLaunchKernelGGL((k_update_mr<float, K>), dim3(vg), dim3(kBlock), 0, stream, (int)n,
                        (const double *)p_new, (const double *)batch.q.p, batch.x.p, batch.r.p,
                        batch.y32.p, batch.partials.p, batch.bs);
   } else {
-    hipLaunchKernelGGL((k_spmv_p_mr<double, K>), dim3(sg), dim3(kBlock), 0, stream, (int)n,
-                       arp.p, aci.p, av.p, (const double *)batch.z64.p, (const double *)p_old,
-                       p_new, batch.q.p, (const double *)batch.r.p, batch.partials.p, batch.bs);
+    hipLaunchKernelGGL((k_p_update_mr<double, K>), dim3(vg), dim3(kBlock), 0, stream, (int)n,
+                       (const double *)batch.z64.p, (const double *)p_old, p_new, batch.bs);
+    hipLaunchKernelGGL((k_spmv_p_mr<K>), dim3(sg), dim3(kBlock), 0, stream, (int)n, arp.p, aci.p,
+                       av.p, (const double *)p_new, batch.q.p, (const double *)batch.r.p,
+                       batch.partials.p, batch.bs);
     if (ev) (void)hipEventRecord(ev[3], stream);
     hipLaunchKernelGGL((k_update_mr<double, K>), dim3(vg), dim3(kBlock), 0, stream, (int)n,
                        (const double *)p_new, (const double *)batch.q.p, batch.x.p, batch.r.p,
@@ -1175,11 +1200,7 @@ int rchol_amd_ctx::pcg_batch(const double *d_b, int ncols, double tol, int maxit
   }
   if (batch.hbs->err)
     return stall(batch.hbs->err);
-  const int rows_per_block = (kBlock / 64) * (64 / K);
-  int sg = (int)std::max<size_t>(
-      1, std::min<size_t>((n + rows_per_block - 1) / rows_per_block, (size_t)ncu * kSpmvMrBlocksPerCu));
-  if (sg > 8) sg = (sg + 7) / 8 * 8;  // whole XCD rounds for the row walk
-  hipLaunchKernelGGL((k_spmv_res_mr<K>), dim3(sg), dim3(kBlock), 0, stream, (int)n, arp.p, aci.p,
+  hipLaunchKernelGGL((k_spmv_res_mr<K>), dim3(spmv_mr_grid(K)), dim3(kBlock), 0, stream, (int)n, arp.p, aci.p,
                      av.p, (const double *)batch.x.p, d_b, batch.res.p, batch.partials.p, batch.bs);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(ev1, stream));

@@ -61,7 +61,7 @@ typedef struct rchol_amd_ctx rchol_amd_ctx;
                                          orders) instead of level by level.  -1 (default):
                                          planned at upload_G when the factor has many narrow
                                          levels, used when its estimate beats the level
-                                         schedule; 0: never; 1: always (planned at the next
+                                         schedule, merged or not; 0: never; 1: always (planned at the next
                                          upload_G; set before it) */
 #define RCHOL_AMD_OPT_WAIT_TICKS 11   /* bound of every dependency / residency wait, in
                                          ticks of the 100 MHz wall clock, for the GPU of
@@ -70,7 +70,7 @@ typedef struct rchol_amd_ctx rchol_amd_ctx;
                                          longer waits into RCHOL_AMD_ESTALL: for testing
                                          the error path */
 #define RCHOL_AMD_OPT_MERGE 12        /* 1 (default): the next upload_G merges consecutive narrow
-                                         levels of the single-right-hand-side sweeps into
+                                         levels of the sweeps (one to eight columns) into
                                          groups of one handshake each, where the factor's
                                          signs allow it; 0: it does not (a shorter upload, for
                                          a factor that is used once) */

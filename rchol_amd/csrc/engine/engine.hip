@@ -455,6 +455,7 @@ struct rchol_amd_ctx {
   int chunk_mode = -1;      // RCHOL_AMD_OPT_CHUNKED
   int merge_levels = 1;     // RCHOL_AMD_OPT_MERGE
   bool chunk_auto = false;  // the upload's own choice (chunk_mode -1)
+  double chunk_est_us = 0.0;  // both sweeps in chunks, planned with the last factor
   bool use_chunks = false;  // single-RHS sweeps run k_sptrsv_chunk
   int lds_max = 0;          // LDS bytes a workgroup may allocate
   int chunk_grid = 0;       // workgroups of the chunked sweeps
@@ -1769,11 +1770,15 @@ int chunk_launch_setup(rchol_amd_ctx *c, size_t lds) {
   return RCHOL_AMD_OK;
 }
 
+// Many narrow levels: the factors that chunks and deep level groups are for.
+bool is_deep(size_t n, int nlf, int nlb) {
+  const int nl = std::max(nlf, nlb);
+  return nl >= kChunkMinLevels && (double)n / nl < kChunkMaxMeanWidth;
+}
+
 // Whether the upload plans the chunked sweeps.
 bool plans_chunks(const rchol_amd_ctx *c, size_t n, int nlf, int nlb) {
-  const int nl = std::max(nlf, nlb);
-  const bool deep = nl >= kChunkMinLevels && (double)n / nl < kChunkMaxMeanWidth;
-  return c->chunk_mode == 1 || (c->chunk_mode == -1 && deep);
+  return c->chunk_mode == 1 || (c->chunk_mode == -1 && is_deep(n, nlf, nlb));
 }
 
 // Plan (and, when chosen, upload) the chunked sweeps of a factor whose
@@ -1796,7 +1801,8 @@ int setup_chunks(rchol_amd_ctx *c, size_t n, HostSweep &hf, HostSweep &hb, int n
   HostChunks pf, pb;
   plan_chunks(hf, (int)n, bnd, false, pf);
   plan_chunks(hb, (int)n, bnd, true, pb);
-  c->chunk_auto = pf.est_us + pb.est_us < (nlf + nlb) * kLevelUs;
+  c->chunk_est_us = pf.est_us + pb.est_us;
+  c->chunk_auto = c->chunk_est_us < (nlf + nlb) * kLevelUs;
   if (c->chunk_mode == -1 && !c->chunk_auto) return RCHOL_AMD_OK;
   int rc = upload_chunks(c->fwd.ch, pf, precision);
   if (!rc) rc = upload_chunks(c->bwd.ch, pb, precision);
@@ -1845,10 +1851,11 @@ int rchol_amd_upload_G(rchol_amd_ctx *c, size_t n, const size_t *colPtr, const s
       if (t.joinable()) t.join();
     }
   } join{planner};
-  if (c->merge_levels && !plans_chunks(c, n, nlf, nlb)) {
+  if (c->merge_levels && c->chunk_mode != 1) {
     auto plan = [&]() {
+      const MergeLimits lim = merge_limits(is_deep(n, nlf, nlb), n, nnz);
       for (int k = 0; k < 2; k++) try {
-          plan_merge(k ? hb : hf, n, mplan[k]);
+          plan_merge(k ? hb : hf, n, lim, mplan[k]);
         } catch (const std::exception &) {  // no memory or threads for it: the plain levels
           mplan[k] = MergePlan();
         }
@@ -1909,7 +1916,18 @@ int rchol_amd_upload_G(rchol_amd_ctx *c, size_t n, const size_t *colPtr, const s
   };
   int rc = up(c->fwd, hf);
   if (!rc) rc = up(c->bwd, hb);
+  if (!rc) rc = setup_chunks(c, n, hf, hb, nlf, nlb, precision);
   if (planner.joinable()) planner.join();
+  // A deep factor has both plans: the merged levels when they are estimated
+  // faster, the chunks' estimate raised to what they take (estimated / taken,
+  // both sweeps, ms: merged 0.16 / 0.25 at 24^3 natural, 0.55 / 1.10 at static
+  // 40^3, 1.98 / 2.12 at 64^3, 2.86 / 2.96 at 72^3; chunks 0.49 / 0.58,
+  // 0.92 / 1.46, 2.01 / 3.44 and 2.64 / 4.87)
+  if (c->use_chunks && c->chunk_mode == -1 && mplan[0].any() && mplan[1].any() &&
+      mplan[0].est_us + mplan[1].est_us < 1.5 * c->chunk_est_us) {
+    c->chunk_auto = false;
+    c->use_chunks = false;
+  }
   if (!rc) rc = up_merged(c->fwd, mplan[0]);
   if (!rc) rc = up_merged(c->bwd, mplan[1]);
   if (rc) return rc;
@@ -1919,8 +1937,6 @@ int rchol_amd_upload_G(rchol_amd_ctx *c, size_t n, const size_t *colPtr, const s
   c->g_gen++;
   const double t2 = host_ms();
   rc = c->size_trsv_grid();
-  if (rc) return rc;
-  rc = setup_chunks(c, n, hf, hb, nlf, nlb, precision);
   if (rc) return rc;
   c->hasG = true;
   c->stats.chunked = c->use_chunks ? 1 : 0;
@@ -2660,8 +2676,9 @@ int rchol_amd_merge_apply_host(size_t n, const size_t *colPtr, const size_t *row
   int rc = analyze_factor(n, colPtr, rowIdx, val, hf, hb, nlf, nlb);
   if (rc) return rc;
   MergePlan pf, pb;
-  plan_merge(hf, n, pf);
-  plan_merge(hb, n, pb);
+  const MergeLimits lim = merge_limits(is_deep(n, nlf, nlb), n, colPtr[n]);
+  plan_merge(hf, n, lim, pf);
+  plan_merge(hb, n, lim, pb);
   std::vector<double> y(n);
   rc = simulate_merge(hf, pf, n, r, y.data());
   if (!rc) rc = simulate_merge(hb, pb, n, y.data(), z);

@@ -30,16 +30,35 @@
 #ifndef RCHOL_AMD_MERGE_PS
 #define RCHOL_AMD_MERGE_PS 5.0
 #endif
+constexpr double kHopUs = RCHOL_AMD_MERGE_HOP;
+constexpr double kEntryUs = RCHOL_AMD_MERGE_PS * 1e-6;
+// How far a level is merged: microseconds of entries that merging may add to
+// it, mean entries of its merged rows.
+struct MergeLimits {
+  double cap_us, len;
+};
 #ifndef RCHOL_AMD_MERGE_CAP
 #define RCHOL_AMD_MERGE_CAP 0.2
 #endif
 #ifndef RCHOL_AMD_MERGE_LEN
 #define RCHOL_AMD_MERGE_LEN 1024
 #endif
-constexpr double kHopUs = RCHOL_AMD_MERGE_HOP;
-constexpr double kEntryUs = RCHOL_AMD_MERGE_PS * 1e-6;
-constexpr double kMergeCapUs = RCHOL_AMD_MERGE_CAP;
-constexpr double kMergeLen = RCHOL_AMD_MERGE_LEN;
+// A deep factor (thousands of narrow levels) has few rows per level: deeper
+// groups, to rows that grow at most kDeepGrowth-fold on average (24^3 in
+// natural order, 2929 levels, FP64: 48-fold 7.5 ms per solve and 40 ms of
+// planning, 96-fold 5.7 and 55; static 64^3, 8216 levels: 54 and 51 ms).
+#ifndef RCHOL_AMD_MERGE_DEEP_CAP
+#define RCHOL_AMD_MERGE_DEEP_CAP 0.05
+#endif
+#ifndef RCHOL_AMD_MERGE_DEEP_LEN
+#define RCHOL_AMD_MERGE_DEEP_LEN 2048
+#endif
+constexpr double kDeepGrowth = 96.0;
+MergeLimits merge_limits(bool deep, size_t n, size_t nnz) {
+  if (!deep) return {RCHOL_AMD_MERGE_CAP, RCHOL_AMD_MERGE_LEN};
+  return {RCHOL_AMD_MERGE_DEEP_CAP,
+          std::min<double>(RCHOL_AMD_MERGE_DEEP_LEN, kDeepGrowth * (double)nnz / (double)n)};
+}
 
 struct MergePlan {
   std::vector<int> gptr;  // group g: levels [gptr[g], gptr[g + 1])
@@ -52,53 +71,54 @@ struct MergePlan {
   bool any() const { return m1 > m0; }
 };
 
-// Column -> value map of one row under elimination, in insertion order
-// (open addressing; `at` lists the used places so that clearing costs the
-// row's length).
+// Column -> value map of one row under elimination, in insertion order.  Up to
+// kDirectMap rows a place per column; beyond, open addressing.  `at` lists the
+// used places so that clearing costs the row's length.
+constexpr size_t kDirectMap = (size_t)1 << 20;
 struct RowMap {
-  std::vector<int> key, pos, at;  // key[p] == c: column c is cols[pos[p]]
-  std::vector<int> cols;
+  struct Place {
+    int key, pos;  // key == c: column c is cols[pos]
+  };
+  std::vector<Place> tab;
+  std::vector<int> at, cols;
   std::vector<double> vals;
+  bool direct;
   size_t mask = 1023;
-  RowMap() : key(1024, -1), pos(1024) {}
+  explicit RowMap(size_t n) : tab(n <= kDirectMap ? n : 1024, Place{-1, 0}), direct(n <= kDirectMap) {}
   size_t find(int c) const {
+    if (direct) return (size_t)c;
     size_t p = (size_t)((unsigned)c * 2654435761u >> 7) & mask;
-    while (key[p] != -1 && key[p] != c) p = (p + 1) & mask;
+    while (tab[p].key != -1 && tab[p].key != c) p = (p + 1) & mask;
     return p;
   }
   void clear() {
-    for (int p : at) key[p] = -1;
+    for (int p : at) tab[p].key = -1;
     at.clear();
     cols.clear();
     vals.clear();
   }
-  void put(int c, int k) {
-    const size_t p = find(c);
-    key[p] = c;
-    pos[p] = k;
+  void put(size_t p, int c, int k) {
+    tab[p] = Place{c, k};
     at.push_back((int)p);
   }
   // Adds v to column c and returns its place in cols / vals; fresh: new.
   int add(int c, double v, bool &fresh) {
     const size_t p = find(c);
-    fresh = key[p] == -1;
+    fresh = tab[p].key == -1;
     if (!fresh) {
-      vals[pos[p]] += v;
-      return pos[p];
+      vals[tab[p].pos] += v;
+      return tab[p].pos;
     }
     const int k = (int)cols.size();
     cols.push_back(c);
     vals.push_back(v);
-    if (2 * cols.size() > mask) {
+    if (!direct && 2 * cols.size() > mask) {
       mask = 4 * (mask + 1) - 1;
-      key.assign(mask + 1, -1);
-      pos.resize(mask + 1);
+      tab.assign(mask + 1, Place{-1, 0});
       at.clear();
-      for (int q = 0; q <= k; q++) put(cols[q], q);
+      for (int q = 0; q <= k; q++) put(find(cols[q]), cols[q], q);
     } else {
-      key[p] = c;
-      pos[p] = k;
-      at.push_back((int)p);
+      put(p, c, k);
     }
     return k;
   }
@@ -110,6 +130,7 @@ struct RowElim {
   RowMap map;
   std::vector<std::vector<int>> bucket;  // map positions of the dependencies per level - l0
   int depth = 0;
+  explicit RowElim(size_t n) : map(n) {}
 
   // Eliminate row i (level m) of the group that starts at level l0.  With
   // values: map holds every column's merged coefficient (dependencies inside
@@ -173,12 +194,14 @@ bool merge_signs(const HostSweep &h, size_t n) {
 // that level's rows, merged, stay within kMergeLen entries on average and the
 // entries that merging adds to the level cost less than kMergeCapUs of the
 // handshake they save.  Merged lengths come from a sample of the level's
-// rows.
+// rows.  Neighbouring groups are about as deep as each other, so the search
+// starts at the depth of the last one and goes up or down from there.
 constexpr int kMergeSample = 6;
 
-void plan_groups(const HostSweep &h, const IntVec &lev, int a, int b, std::vector<int> &gptr) {
+void plan_groups(const HostSweep &h, const IntVec &lev, int a, int b, const MergeLimits &lim,
+                 std::vector<int> &gptr) {
   const std::vector<int> &lp = h.level_ptr;
-  RowElim el;
+  RowElim el(h.nat_rp.size() - 1);
   auto mean_merged = [&](int m, int l0, double &merged, double &plain) {
     const int w = lp[m + 1] - lp[m], k = std::min(w, kMergeSample);
     merged = plain = 0.0;
@@ -190,25 +213,32 @@ void plan_groups(const HostSweep &h, const IntVec &lev, int a, int b, std::vecto
     merged /= k;
     plain /= k;
   };
+  // whether the group [l, e) may hold its last levels (an eighth of them)
+  auto fits = [&](int l, int e) {
+    double merged, plain, worst = 0.0;
+    mean_merged(e - 1, l, merged, plain);
+    for (int q = e - std::max(1, (e - l) / 9); q < e; q++)
+      worst = std::max(worst, (double)(lp[q + 1] - lp[q]));
+    return merged <= lim.len && (merged - plain) * worst * kEntryUs <= lim.cap_us;
+  };
+  int depth = 1;
   for (int l = a; l < b;) {
-    int e = l + 1;
-    while (e < b) {
-      // look `step` levels ahead in a group that is already deep
-      const int step = std::max(1, (e - l) / 8);
-      const int m = std::min(b, e + step) - 1;
-      double merged, plain, worst = 0.0;
-      mean_merged(m, l, merged, plain);
-      for (int q = e; q <= m; q++) worst = std::max(worst, (double)(lp[q + 1] - lp[q]));
-      if (merged > kMergeLen || (merged - plain) * worst * kEntryUs > kMergeCapUs) break;
-      e = m + 1;
+    const int guess = std::min(b, l + depth);
+    int e = guess;
+    while (e - l > 1 && !fits(l, e)) e = std::max(l + 1, e - std::max(1, (e - l) / 8));
+    while (e >= guess && e < b) {
+      const int m = std::min(b, e + std::max(1, (e - l) / 8));
+      if (!fits(l, m)) break;
+      e = m;
     }
+    depth = e - l;
     gptr.push_back(l);
     l = e;
   }
 }
 
 // Merge plan of one sweep (empty when no two levels are worth merging).
-void plan_merge(const HostSweep &h, size_t n, MergePlan &out) {
+void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan &out) {
   const std::vector<int> &lp = h.level_ptr;
   const int nl = h.nlevels;
   out = MergePlan();
@@ -219,16 +249,18 @@ void plan_merge(const HostSweep &h, size_t n, MergePlan &out) {
     for (size_t l = l0; l < l1; l++)
       for (int s = lp[l]; s < lp[l + 1]; s++) lev[h.slot_row[s]] = (int)l;
   }, 32);
-  // groups, in runs of levels of about equal entries planned in parallel (a
-  // fixed number, so the plan does not depend on the threads)
+  // groups, in runs of levels of about equal work planned in parallel (a
+  // fixed number, so the plan does not depend on the threads): half of a
+  // run's share counted in entries, half in levels, since the narrow levels
+  // hold few entries and most of the planning
   {
     const long long total = h.rp[n];
     const int S = (int)std::max<long long>(1, std::min<long long>({16, total / 500000, nl / 8}));
     std::vector<int> cut{0};
     for (int k = 1; k < S; k++) {
-      const int goal = (int)(total * k / S);
+      const double goal = (double)k / S;
       int l = cut.back();
-      while (l < nl && h.rp[lp[l]] < goal) l++;
+      while (l < nl && 0.5 * ((double)h.rp[lp[l]] / total + (double)l / nl) < goal) l++;
       if (l > cut.back() && l < nl) cut.push_back(l);
     }
     cut.push_back(nl);
@@ -236,7 +268,7 @@ void plan_merge(const HostSweep &h, size_t n, MergePlan &out) {
     std::vector<std::vector<int>> part(R);
     std::atomic<int> next{0};
     par_run(std::min(host_threads(), R), [&](int) {
-      for (int k; (k = next.fetch_add(1)) < R;) plan_groups(h, lev, cut[k], cut[k + 1], part[k]);
+      for (int k; (k = next.fetch_add(1)) < R;) plan_groups(h, lev, cut[k], cut[k + 1], lim, part[k]);
     });
     for (auto &p : part) out.gptr.insert(out.gptr.end(), p.begin(), p.end());
     out.gptr.push_back(nl);
@@ -273,7 +305,7 @@ void plan_merge(const HostSweep &h, size_t n, MergePlan &out) {
   std::atomic<bool> over{false};  // a limit was passed: no plan
   const long long most = std::min<long long>(kMergeMaxGrowth * (h.rp[n] + (long long)n), INT_MAX / 2);
   auto merge_rows = [&]() {
-    RowElim el;
+    RowElim el(n);
     Block o;
     std::vector<unsigned long long> key;  // level | column | map position
     for (int b; (b = next.fetch_add(1)) < B && !over;) {

@@ -33,10 +33,12 @@
 constexpr double kHopUs = RCHOL_AMD_MERGE_HOP;
 constexpr double kEntryUs = RCHOL_AMD_MERGE_PS * 1e-6;
 // How far a level is merged: microseconds of entries that merging may add to
-// it, mean entries of its merged rows.
+// it, mean entries of its merged rows; most levels of a sweep that is merged.
 struct MergeLimits {
   double cap_us, len;
+  int levels;
 };
+constexpr int kMergeMaxLevels = 1 << 20;  // (fits the sort key of a merged entry)
 #ifndef RCHOL_AMD_MERGE_CAP
 #define RCHOL_AMD_MERGE_CAP 0.2
 #endif
@@ -47,6 +49,9 @@ struct MergeLimits {
 // groups, to rows that grow at most kDeepGrowth-fold on average (24^3 in
 // natural order, 2929 levels, FP64: 48-fold 7.5 ms per solve and 40 ms of
 // planning, 96-fold 5.7 and 55; static 64^3, 8216 levels: 54 and 51 ms).
+// Planning grows with the levels and stays out beyond kDeepMaxLevels (static
+// 72^3, 10817 levels: 0.24 s; 256^3, 104163 levels: 4.5 s, for sweeps that the
+// chunks win).
 #ifndef RCHOL_AMD_MERGE_DEEP_CAP
 #define RCHOL_AMD_MERGE_DEEP_CAP 0.05
 #endif
@@ -54,10 +59,12 @@ struct MergeLimits {
 #define RCHOL_AMD_MERGE_DEEP_LEN 2048
 #endif
 constexpr double kDeepGrowth = 96.0;
+constexpr int kDeepMaxLevels = 16384;
 MergeLimits merge_limits(bool deep, size_t n, size_t nnz) {
-  if (!deep) return {RCHOL_AMD_MERGE_CAP, RCHOL_AMD_MERGE_LEN};
+  if (!deep) return {RCHOL_AMD_MERGE_CAP, RCHOL_AMD_MERGE_LEN, kMergeMaxLevels};
   return {RCHOL_AMD_MERGE_DEEP_CAP,
-          std::min<double>(RCHOL_AMD_MERGE_DEEP_LEN, kDeepGrowth * (double)nnz / (double)n)};
+          std::min<double>(RCHOL_AMD_MERGE_DEEP_LEN, kDeepGrowth * (double)nnz / (double)n),
+          kDeepMaxLevels};
 }
 
 struct MergePlan {
@@ -164,7 +171,7 @@ struct RowElim {
 
 // Sort key of a merged entry: level (20 bits) | column (31) | place (13).
 constexpr int kKeyPos = 13, kKeyLevel = 44;
-constexpr int kMergeMaxLevels = 1 << 20;
+static_assert(kKeyLevel + 20 == 64 && kMergeMaxLevels == 1 << 20, "sort key");
 constexpr int kMergeMaxRow = 1 << kKeyPos;
 // Largest merged coefficient: one beyond it (pivots that differ by tens of
 // orders of magnitude) could overflow where the substitution does not.
@@ -243,7 +250,7 @@ void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan 
   const int nl = h.nlevels;
   out = MergePlan();
   out.gptr.clear();
-  if (nl < 2 || nl > kMergeMaxLevels || !merge_signs(h, n)) return;
+  if (nl < 2 || nl > lim.levels || !merge_signs(h, n)) return;
   IntVec lev(n);
   par_for((size_t)nl, [&](size_t l0, size_t l1) {
     for (size_t l = l0; l < l1; l++)

@@ -274,9 +274,16 @@ void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan 
     const int R = (int)cut.size() - 1;
     std::vector<std::vector<int>> part(R);
     std::atomic<int> next{0};
+    std::atomic<bool> failed{false};  // an exception may not leave a host thread
     par_run(std::min(host_threads(), R), [&](int) {
-      for (int k; (k = next.fetch_add(1)) < R;) plan_groups(h, lev, cut[k], cut[k + 1], lim, part[k]);
+      try {
+        for (int k; (k = next.fetch_add(1)) < R;)
+          plan_groups(h, lev, cut[k], cut[k + 1], lim, part[k]);
+      } catch (const std::bad_alloc &) {
+        failed = true;
+      }
     });
+    if (failed) return;
     for (auto &p : part) out.gptr.insert(out.gptr.end(), p.begin(), p.end());
     out.gptr.push_back(nl);
   }

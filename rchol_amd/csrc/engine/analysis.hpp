@@ -2,8 +2,8 @@
 // levels of the forward and the backward sweep, rows in level ("slot")
 // order and their off-diagonal entries in that order.  Plain C++ (no HIP):
 // included by engine.hip inside its anonymous namespace, after fail() and
-// kTaskRows, and after <algorithm>, <atomic>, <chrono>, <memory>, <mutex>,
-// <thread>, <vector> and <sys/mman.h>.
+// kTaskRows, and after <algorithm>, <atomic>, <chrono>, <exception>, <memory>,
+// <mutex>, <thread>, <vector> and <sys/mman.h>.
 //
 // Every pass is parallel over host threads and walks the factor in its own
 // (nested-dissection) order, so the level reads and the scattered writes of
@@ -116,18 +116,36 @@ double host_ms() {
       .count();
 }
 
-// f(t) for t in [0, T): T-1 new threads, the caller's thread runs t = 0.
+// f(t) for t in [0, T): T-1 new threads, the caller's thread runs t = 0 and,
+// after it, every t that no thread could be started for.  All threads are
+// joined before the first exception of any of them goes on to the caller.
 template <typename F>
 void par_run(int T, F &&f) {
   if (T <= 1) {
     f(0);
     return;
   }
+  std::mutex mu;
+  std::exception_ptr first;
+  auto run = [&](int t) {
+    try {
+      f(t);
+    } catch (...) {
+      std::lock_guard<std::mutex> g(mu);
+      if (!first) first = std::current_exception();
+    }
+  };
   std::vector<std::thread> th;
   th.reserve(T - 1);
-  for (int t = 1; t < T; t++) th.emplace_back([&f, t]() { f(t); });
-  f(0);
+  int started = 1;
+  try {
+    for (; started < T; started++) th.emplace_back([&run, t = started]() { run(t); });
+  } catch (const std::exception &) {  // no thread or no memory for one
+  }
+  run(0);
+  for (int t = started; t < T; t++) run(t);
   for (auto &x : th) x.join();
+  if (first) std::rethrow_exception(first);
 }
 
 // f(lo, hi) over [0, n) in contiguous chunks, one per thread (chunks of at
@@ -185,7 +203,8 @@ std::vector<size_t> column_ranges(size_t n, const size_t *colPtr, int T) {
 // Tasks of a dependency graph on a pool of T threads: task v may run once
 // every task u with an edge u -> v has finished (succ_ptr/succ: the edges
 // out of each task, indeg: edges into it).  Ready tasks wait on a shared
-// stack; piece(t, v) runs task v on thread t.
+// stack; piece(t, v) runs task v on thread t.  A piece that throws ends the
+// pool: the tasks after it would never become ready.
 template <typename F>
 void run_dag(int V, const std::vector<int> &succ_ptr, const std::vector<int> &succ,
              std::vector<int> &indeg, int T, F &&piece) {
@@ -194,7 +213,8 @@ void run_dag(int V, const std::vector<int> &succ_ptr, const std::vector<int> &su
   for (int v = 0; v < V; v++)
     if (indeg[v] == 0) ready.push_back(v);
   std::atomic<int> left{V};
-  par_run(T, [&](int t) {
+  std::atomic<bool> failed{false};
+  auto work = [&](int t) {
     for (;;) {
       int v = -1;
       {
@@ -205,7 +225,7 @@ void run_dag(int V, const std::vector<int> &succ_ptr, const std::vector<int> &su
         }
       }
       if (v < 0) {
-        if (left.load(std::memory_order_acquire) == 0) return;
+        if (left.load(std::memory_order_acquire) == 0 || failed) return;
         std::this_thread::yield();
         continue;
       }
@@ -218,6 +238,14 @@ void run_dag(int V, const std::vector<int> &succ_ptr, const std::vector<int> &su
         }
       }
       left.fetch_sub(1, std::memory_order_acq_rel);
+    }
+  };
+  par_run(T, [&](int t) {
+    try {
+      work(t);
+    } catch (...) {
+      failed = true;
+      throw;
     }
   });
 }

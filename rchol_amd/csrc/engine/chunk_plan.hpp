@@ -21,13 +21,9 @@ template <typename F>
 void par_each(size_t n, F &&f) {
   const size_t T = std::min<size_t>((size_t)host_threads(), n);
   std::atomic<size_t> next{0};
-  auto run = [&]() {
+  par_run((int)T, [&](int) {
     for (size_t i; (i = next.fetch_add(1)) < n;) f(i);
-  };
-  std::vector<std::thread> th;
-  for (size_t t = 1; t < T; t++) th.emplace_back(run);
-  run();
-  for (auto &x : th) x.join();
+  });
 }
 constexpr int kChunkWindow = 64;
 

@@ -57,6 +57,12 @@ int fail(int code, const char *fmt, ...) {
   return code;
 }
 
+// An exception (host memory, in the analysis or a plan of a factor) may not
+// leave a C entry point: the handler of those that run them.
+int host_failure(const std::exception &e) {
+  return fail(RCHOL_AMD_EHIP, "host failure: %s", e.what());
+}
+
 // The error flag of a sweep as a message: bit 0 a dependency wait hit its
 // bound, bit 1 a schedule held a task kind the kernel does not run, bit 2
 // the persistent grid's workgroups were not all resident at once.
@@ -1824,7 +1830,7 @@ int setup_chunks(rchol_amd_ctx *c, size_t n, HostSweep &hf, HostSweep &hb, int n
 extern "C" {
 
 int rchol_amd_upload_G(rchol_amd_ctx *c, size_t n, const size_t *colPtr, const size_t *rowIdx,
-                       const double *val, int precision) {
+                       const double *val, int precision) try {
   if (!c || !colPtr || !rowIdx || !val) return fail(RCHOL_AMD_EINVAL, "null argument");
   if (precision != RCHOL_AMD_FP64 && precision != RCHOL_AMD_FP32)
     return fail(RCHOL_AMD_EINVAL, "unknown precision %d", precision);
@@ -1953,6 +1959,8 @@ int rchol_amd_upload_G(rchol_amd_ctx *c, size_t n, const size_t *colPtr, const s
   c->stats.bwd_levels = nlb;
   c->stats.g_precision = precision;
   return RCHOL_AMD_OK;
+} catch (const std::exception &e) {
+  return host_failure(e);
 }
 
 int rchol_amd_set_option(rchol_amd_ctx *c, int key, double value) {
@@ -2474,7 +2482,7 @@ int rchol_amd_copy_probe(rchol_amd_ctx *c, size_t bytes, int reps, double *gbs, 
 
 
 int rchol_amd_analyze_G(size_t n, const size_t *colPtr, const size_t *rowIdx, const double *val,
-                        int serial_width, rchol_amd_schedule *out) {
+                        int serial_width, rchol_amd_schedule *out) try {
   if (!colPtr || !rowIdx || !val || !out) return fail(RCHOL_AMD_EINVAL, "null argument");
   if (n == 0 || n > kIdxMax) return fail(RCHOL_AMD_ERANGE, "n=%zu outside [1, 2^31)", n);
   if (colPtr[0] != 0) return fail(RCHOL_AMD_EINVAL, "colPtr[0] must be 0");
@@ -2503,6 +2511,8 @@ int rchol_amd_analyze_G(size_t n, const size_t *colPtr, const size_t *rowIdx, co
     memcpy(out->proxy[k], h[k].proxy.data(), n * sizeof(unsigned short));
   }
   return RCHOL_AMD_OK;
+} catch (const std::exception &e) {
+  return host_failure(e);
 }
 
 }  // extern "C"
@@ -2633,7 +2643,7 @@ extern "C" {
 
 int rchol_amd_chunk_apply_host(size_t n, const size_t *colPtr, const size_t *rowIdx,
                                const double *val, int max_rows, const double *r, double *z,
-                               int *counts, long long *rounds, double *est_us) {
+                               int *counts, long long *rounds, double *est_us) try {
   if (!colPtr || !rowIdx || !val || !r || !z) return fail(RCHOL_AMD_EINVAL, "null argument");
   if (n == 0 || n > kIdxMax) return fail(RCHOL_AMD_ERANGE, "n=%zu outside [1, 2^31)", n);
   if (colPtr[0] != 0) return fail(RCHOL_AMD_EINVAL, "colPtr[0] must be 0");
@@ -2663,11 +2673,13 @@ int rchol_amd_chunk_apply_host(size_t n, const size_t *colPtr, const size_t *row
     est_us[1] = pb.est_us;
   }
   return RCHOL_AMD_OK;
+} catch (const std::exception &e) {
+  return host_failure(e);
 }
 
 int rchol_amd_merge_apply_host(size_t n, const size_t *colPtr, const size_t *rowIdx,
                                const double *val, const double *r, double *z, int *groups,
-                               long long *entries, double *est_us) {
+                               long long *entries, double *est_us) try {
   if (!colPtr || !rowIdx || !val || !r || !z) return fail(RCHOL_AMD_EINVAL, "null argument");
   if (n == 0 || n > kIdxMax) return fail(RCHOL_AMD_ERANGE, "n=%zu outside [1, 2^31)", n);
   if (colPtr[0] != 0) return fail(RCHOL_AMD_EINVAL, "colPtr[0] must be 0");
@@ -2691,6 +2703,8 @@ int rchol_amd_merge_apply_host(size_t n, const size_t *colPtr, const size_t *row
     if (est_us) est_us[k] = p[k]->est_us;
   }
   return RCHOL_AMD_OK;
+} catch (const std::exception &e) {
+  return host_failure(e);
 }
 
 void rchol_amd_schedule_free(rchol_amd_schedule *s) {

@@ -274,16 +274,10 @@ void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan 
     const int R = (int)cut.size() - 1;
     std::vector<std::vector<int>> part(R);
     std::atomic<int> next{0};
-    std::atomic<bool> failed{false};  // an exception may not leave a host thread
     par_run(std::min(host_threads(), R), [&](int) {
-      try {
-        for (int k; (k = next.fetch_add(1)) < R;)
-          plan_groups(h, lev, cut[k], cut[k + 1], lim, part[k]);
-      } catch (const std::bad_alloc &) {
-        failed = true;
-      }
+      for (int k; (k = next.fetch_add(1)) < R;)
+        plan_groups(h, lev, cut[k], cut[k + 1], lim, part[k]);
     });
-    if (failed) return;
     for (auto &p : part) out.gptr.insert(out.gptr.end(), p.begin(), p.end());
     out.gptr.push_back(nl);
   }
@@ -318,7 +312,7 @@ void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan 
   std::atomic<long long> total{0};
   std::atomic<bool> over{false};  // a limit was passed: no plan
   const long long most = std::min<long long>(kMergeMaxGrowth * (h.rp[n] + (long long)n), INT_MAX / 2);
-  auto merge_rows = [&]() {
+  par_run(std::min(host_threads(), std::max(1, B / 4)), [&](int) {
     RowElim el(n);
     Block o;
     std::vector<unsigned long long> key;  // level | column | map position
@@ -364,13 +358,6 @@ void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan 
       blk[b].ci.assign(o.ci.begin(), o.ci.end());
       blk[b].cv.assign(o.cv.begin(), o.cv.end());
       if (total.fetch_add((long long)o.ci.size()) + (long long)o.ci.size() > most) over = true;
-    }
-  };
-  par_run(std::min(host_threads(), std::max(1, B / 4)), [&](int) {
-    try {
-      merge_rows();
-    } catch (const std::bad_alloc &) {
-      over = true;
     }
   });
   if (over) {

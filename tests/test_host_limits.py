@@ -1,5 +1,6 @@
 """The host analysis and plans of a factor when the process is short of threads
-(the work is done by those that start), run in a process with the limit."""
+(the work is done by those that start) or of memory (an error, or the result),
+run in a process with the limit."""
 import os
 import resource
 import subprocess
@@ -37,6 +38,34 @@ print("threads", len(started), flush=True)
 z = merge_apply_host(Gs, d["r"])
 c = chunk_apply_host(Gs, d["r"])
 np.savez(sys.argv[2], zm=z[0], groups=z[1], ents=z[2], zc=c[0], counts=c[1])
+"""
+
+
+MEMORY_CHILD = """
+import resource
+import sys
+import numpy as np
+from rchol_amd import solver as S
+
+d = np.load(sys.argv[1])
+Gs = (d["cp"], d["ri"], d["v"])
+r = d["r"]
+e = np.array([0, 1, 2], dtype=np.uint64)
+call = {"merge": lambda G, b: S.merge_apply_host(G, b)[0],
+        "chunk": lambda G, b: S.chunk_apply_host(G, b)[0],
+        "analyze": lambda G, b: S.analyze(G)["fwd"]["slot_row"]}[sys.argv[3]]
+call((e, e[:2], np.ones(2)), np.ones(2))  # everything is loaded
+for room in sys.argv[2].split(","):
+    size = next(int(l.split()[1]) << 10 for l in open("/proc/self/status") if l.startswith("VmSize"))
+    resource.setrlimit(resource.RLIMIT_AS, (size + (int(room) << 20), resource.RLIM_INFINITY))
+    z = None
+    try:
+        z = call(Gs, r)
+    except (RuntimeError, MemoryError) as err:
+        said = str(err)
+    resource.setrlimit(resource.RLIMIT_AS, (resource.RLIM_INFINITY, resource.RLIM_INFINITY))
+    print("refused " + said[:60] if z is None else
+          "done %r" % float(np.dot(z, np.arange(1, z.size + 1) / z.size)), flush=True)
 """
 
 
@@ -81,3 +110,17 @@ def test_plans_without_all_their_threads(system, tmp_path, threads):
     np.testing.assert_array_equal(d["zc"], zc)
     assert d["groups"].tolist() == groups and d["ents"].tolist() == ents
     assert d["counts"].tolist() == counts
+
+
+@pytest.mark.parametrize("what", ["merge", "chunk", "analyze"])
+def test_plans_without_enough_memory(system, what):
+    """An allocation that fails is an error of the call, wherever it falls (one
+    thread: the C library itself ends a process that has no room for a new
+    thread's own data)."""
+    env = dict(os.environ, OMP_NUM_THREADS="1", OPENBLAS_NUM_THREADS="1", PYTHONPATH=ROOT)
+    p = subprocess.run([sys.executable, "-c", MEMORY_CHILD, system[0], "4,24,60,100,140,4000", what],
+                       env=env, cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert p.returncode == 0, (p.returncode, p.stdout, p.stderr)
+    said = p.stdout.splitlines()
+    assert len(said) == 6 and said[0].startswith("refused") and said[-1].startswith("done")
+    assert all(s.startswith("refused") or s == said[-1] for s in said)

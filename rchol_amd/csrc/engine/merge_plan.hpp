@@ -176,9 +176,12 @@ constexpr int kMergeMaxRow = 1 << kKeyPos;
 // Largest merged coefficient: one beyond it (pivots that differ by tens of
 // orders of magnitude) could overflow where the substitution does not.
 constexpr double kMergeMaxAbs = 1e30;
-// Most merged entries of a sweep, in entries and rows of the factor (the
-// groups' own rule stays far below it).
+// Most merged entries of a sweep, in entries and rows of the factor.  The
+// limit on a group's mean row says nothing of it: a chain of 300 rows, or 604
+// levels of a 32 x 32 grid in natural order, fit one group of rows of several
+// hundred entries.  A plan beyond it is made again with shorter rows.
 constexpr long long kMergeMaxGrowth = 64;
+constexpr double kMergeMinLen = 8;  // rows too short to be worth a plan
 
 // Whether every off-diagonal entry of the sweep has the sign opposite to its
 // row's pivot (or is zero).
@@ -244,18 +247,14 @@ void plan_groups(const HostSweep &h, const IntVec &lev, int a, int b, const Merg
   }
 }
 
-// Merge plan of one sweep (empty when no two levels are worth merging).
-void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan &out) {
+// The groups and merged rows of one sweep within the limits (empty when no two
+// levels are worth merging, or a row cannot be merged).  False: more merged
+// entries than kMergeMaxGrowth allows.
+bool plan_within(const HostSweep &h, size_t n, const IntVec &lev, const MergeLimits &lim,
+                 MergePlan &out) {
   const std::vector<int> &lp = h.level_ptr;
   const int nl = h.nlevels;
   out = MergePlan();
-  out.gptr.clear();
-  if (nl < 2 || nl > lim.levels || !merge_signs(h, n)) return;
-  IntVec lev(n);
-  par_for((size_t)nl, [&](size_t l0, size_t l1) {
-    for (size_t l = l0; l < l1; l++)
-      for (int s = lp[l]; s < lp[l + 1]; s++) lev[h.slot_row[s]] = (int)l;
-  }, 32);
   // groups, in runs of levels of about equal work planned in parallel (a
   // fixed number, so the plan does not depend on the threads): half of a
   // run's share counted in entries, half in levels, since the narrow levels
@@ -282,7 +281,7 @@ void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan 
     out.gptr.push_back(nl);
   }
   const int G = (int)out.gptr.size() - 1;
-  if (G == nl) return;
+  if (G == nl) return true;
   IntVec grp(nl);  // group of each level
   int first = -1, last = -1;
   for (int g = 0; g < G; g++) {
@@ -311,6 +310,7 @@ void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan 
   std::atomic<int> next{0};
   std::atomic<long long> total{0};
   std::atomic<bool> over{false};  // a limit was passed: no plan
+  std::atomic<bool> grown{false};  // that of the merged entries
   const long long most = std::min<long long>(kMergeMaxGrowth * (h.rp[n] + (long long)n), INT_MAX / 2);
   par_run(std::min(host_threads(), std::max(1, B / 4)), [&](int) {
     RowElim el(n);
@@ -357,12 +357,13 @@ void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan 
       }
       blk[b].ci.assign(o.ci.begin(), o.ci.end());
       blk[b].cv.assign(o.cv.begin(), o.cv.end());
-      if (total.fetch_add((long long)o.ci.size()) + (long long)o.ci.size() > most) over = true;
+      if (total.fetch_add((long long)o.ci.size()) + (long long)o.ci.size() > most)
+        over = grown = true;
     }
   });
   if (over) {
     out = MergePlan();
-    return;
+    return !grown;
   }
   par_prefix((size_t)M, [&](size_t s) { return len[s]; }, out.rp);
   out.ci.resize(out.rp[M]);
@@ -379,6 +380,25 @@ void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan 
   for (int s = out.m0; s < out.m1; s++)
     if (len[s - out.m0]) ents -= h.rp[s + 1] - h.rp[s];
   out.est_us = G * kHopUs + ents * kEntryUs;
+  return true;
+}
+
+// Merge plan of one sweep (empty when no two levels are worth merging).
+void plan_merge(const HostSweep &h, size_t n, const MergeLimits &lim, MergePlan &out) {
+  const std::vector<int> &lp = h.level_ptr;
+  const int nl = h.nlevels;
+  out = MergePlan();
+  if (nl < 2 || nl > lim.levels || !merge_signs(h, n)) return;
+  IntVec lev(n);
+  par_for((size_t)nl, [&](size_t l0, size_t l1) {
+    for (size_t l = l0; l < l1; l++)
+      for (int s = lp[l]; s < lp[l + 1]; s++) lev[h.slot_row[s]] = (int)l;
+  }, 32);
+  // too many merged entries: rows of at most the mean that the limit leaves,
+  // then half as long, and so on (each attempt stops at the limit)
+  const double share = (double)kMergeMaxGrowth * ((double)h.rp[n] + (double)n) / (double)n;
+  for (MergeLimits l = lim; l.len >= kMergeMinLen; l.len = std::min(0.5 * l.len, share))
+    if (plan_within(h, n, lev, l, out)) return;
 }
 
 // One sweep as the device runs it: groups in order, a merged row from the

@@ -182,6 +182,7 @@ constexpr double kMergeMaxAbs = 1e30;
 // hundred entries.  A plan beyond it is made again with shorter rows.
 constexpr long long kMergeMaxGrowth = 64;
 constexpr double kMergeMinLen = 8;  // rows too short to be worth a plan
+constexpr int kMergeCuts = 6;
 
 // Whether every off-diagonal entry of the sweep has the sign opposite to its
 // row's pivot (or is zero).
@@ -247,9 +248,99 @@ void plan_groups(const HostSweep &h, const IntVec &lev, int a, int b, const Merg
   }
 }
 
+// Merged rows of the groups out.gptr (grp: each level's group) into out: blocks
+// of slots, each into its own arrays, then in order.  A row's entries:
+// right-hand sides, then values by level and column, so that the latest come
+// last and neighbouring columns are gathered together (in the order the
+// elimination meets them: sweeps 4 to 18% slower).  bad[g]: lowered to the
+// lowest level of group g with a row that cannot be merged (which is left
+// out).  False: more merged entries than kMergeMaxGrowth allows.
+bool merge_rows(const HostSweep &h, size_t n, const IntVec &lev, const IntVec &grp,
+                std::vector<std::atomic<int>> &bad, MergePlan &out) {
+  const int M = out.m1 - out.m0;
+  constexpr int kBlk = 64;
+  const int B = (M + kBlk - 1) / kBlk;
+  struct Block {
+    std::vector<int> ci;
+    std::vector<double> cv;
+  };
+  std::vector<Block> blk(B);
+  IntVec len(M);
+  out.proxy.resize(M);
+  std::atomic<int> next{0};
+  std::atomic<long long> total{0};
+  std::atomic<bool> over{false};  // too many merged entries
+  const long long most = std::min<long long>(kMergeMaxGrowth * (h.rp[n] + (long long)n), INT_MAX / 2);
+  par_run(std::min(host_threads(), std::max(1, B / 4)), [&](int) {
+    RowElim el(n);
+    Block o;
+    std::vector<unsigned long long> key;  // level | column | map position
+    for (int b; (b = next.fetch_add(1)) < B && !over;) {
+      o.ci.clear();
+      o.cv.clear();
+      for (int s = out.m0 + b * kBlk; s < std::min(out.m1, out.m0 + (b + 1) * kBlk); s++) {
+        const int i = h.slot_row[s], g = grp[lev[i]], l0 = out.gptr[g];
+        len[s - out.m0] = 0;
+        out.proxy[s - out.m0] = 0;
+        if (lev[i] == l0) continue;  // reads nothing inside its group: its plain row
+        el.run(h, lev, i, l0, true);
+        const RowMap &m = el.map;
+        bool fits = (int)m.cols.size() <= kMergeMaxRow;
+        for (double v : m.vals) fits &= std::fabs(v) <= kMergeMaxAbs;
+        for (int p = 0; p < (int)m.cols.size(); p++)
+          if (lev[m.cols[p]] >= l0)
+            fits &= std::fabs(m.vals[p] / (*h.nat_diag)[m.cols[p]]) <= kMergeMaxAbs;
+        if (!fits) {
+          for (int l = bad[g]; lev[i] < l && !bad[g].compare_exchange_weak(l, lev[i]);) {
+          }
+          continue;
+        }
+        const size_t at = o.ci.size();
+        key.clear();
+        for (int p = 0; p < (int)m.cols.size(); p++) {
+          const int j = m.cols[p], l = lev[j];
+          if (l >= l0) {
+            o.ci.push_back(-2 - j);
+            o.cv.push_back(m.vals[p] / (*h.nat_diag)[j]);
+          } else {
+            key.push_back(((unsigned long long)l << kKeyLevel) | ((unsigned long long)j << kKeyPos) |
+                          (unsigned)p);
+          }
+        }
+        std::sort(key.begin(), key.end());
+        for (unsigned long long q : key) {
+          const int p = (int)(q & ((1u << kKeyPos) - 1));
+          o.ci.push_back(m.cols[p]);
+          o.cv.push_back(m.vals[p]);
+        }
+        len[s - out.m0] = (int)(o.ci.size() - at);
+        out.proxy[s - out.m0] =
+            row_proxy(g, (int)key.size(), [&](int u) { return grp[(int)(key[u] >> kKeyLevel)]; });
+      }
+      blk[b].ci.assign(o.ci.begin(), o.ci.end());
+      blk[b].cv.assign(o.cv.begin(), o.cv.end());
+      if (total.fetch_add((long long)o.ci.size()) + (long long)o.ci.size() > most) over = true;
+    }
+  });
+  if (over) return false;
+  par_prefix((size_t)M, [&](size_t s) { return len[s]; }, out.rp);
+  out.ci.resize(out.rp[M]);
+  out.cv.resize(out.rp[M]);
+  par_for((size_t)B, [&](size_t b0, size_t b1) {
+    for (size_t b = b0; b < b1; b++) {
+      const int o = out.rp[b * kBlk];
+      std::copy(blk[b].ci.begin(), blk[b].ci.end(), out.ci.begin() + o);
+      std::copy(blk[b].cv.begin(), blk[b].cv.end(), out.cv.begin() + o);
+    }
+  }, 64);
+  return true;
+}
+
 // The groups and merged rows of one sweep within the limits (empty when no two
-// levels are worth merging, or a row cannot be merged).  False: more merged
-// entries than kMergeMaxGrowth allows.
+// levels are worth merging).  A group with rows that cannot be merged (longer
+// than kMergeMaxRow, a coefficient beyond kMergeMaxAbs) is cut where the lowest
+// of them stands, up to kMergeCuts times; what is left of it then stays as its
+// plain levels.  False: more merged entries than kMergeMaxGrowth allows.
 bool plan_within(const HostSweep &h, size_t n, const IntVec &lev, const MergeLimits &lim,
                  MergePlan &out) {
   const std::vector<int> &lp = h.level_ptr;
@@ -280,106 +371,46 @@ bool plan_within(const HostSweep &h, size_t n, const IntVec &lev, const MergeLim
     for (auto &p : part) out.gptr.insert(out.gptr.end(), p.begin(), p.end());
     out.gptr.push_back(nl);
   }
-  const int G = (int)out.gptr.size() - 1;
-  if (G == nl) return true;
   IntVec grp(nl);  // group of each level
-  int first = -1, last = -1;
-  for (int g = 0; g < G; g++) {
-    for (int l = out.gptr[g]; l < out.gptr[g + 1]; l++) grp[l] = g;
-    if (out.gptr[g + 1] - out.gptr[g] > 1) {
-      if (first < 0) first = g;
-      last = g;
+  for (int cuts = 0;; cuts++) {
+    const int G = (int)out.gptr.size() - 1;
+    if (G == nl) {
+      out = MergePlan();
+      return true;
     }
-  }
-  out.m0 = lp[out.gptr[first] + 1];  // a group's first level reads nothing inside it
-  out.m1 = lp[out.gptr[last + 1]];
-  const int M = out.m1 - out.m0;
-  // merged rows: blocks of slots, each into its own arrays, then in order.  A
-  // row's entries: right-hand sides, then values by level and column, so that
-  // the latest come last and neighbouring columns are gathered together (in
-  // the order the elimination meets them: sweeps 4 to 18% slower)
-  constexpr int kBlk = 64;
-  const int B = (M + kBlk - 1) / kBlk;
-  struct Block {
-    std::vector<int> ci;
-    std::vector<double> cv;
-  };
-  std::vector<Block> blk(B);
-  IntVec len(M);
-  out.proxy.resize(M);
-  std::atomic<int> next{0};
-  std::atomic<long long> total{0};
-  std::atomic<bool> over{false};  // a limit was passed: no plan
-  std::atomic<bool> grown{false};  // that of the merged entries
-  const long long most = std::min<long long>(kMergeMaxGrowth * (h.rp[n] + (long long)n), INT_MAX / 2);
-  par_run(std::min(host_threads(), std::max(1, B / 4)), [&](int) {
-    RowElim el(n);
-    Block o;
-    std::vector<unsigned long long> key;  // level | column | map position
-    for (int b; (b = next.fetch_add(1)) < B && !over;) {
-      o.ci.clear();
-      o.cv.clear();
-      for (int s = out.m0 + b * kBlk; s < std::min(out.m1, out.m0 + (b + 1) * kBlk); s++) {
-        const int i = h.slot_row[s], g = grp[lev[i]], l0 = out.gptr[g];
-        len[s - out.m0] = 0;
-        out.proxy[s - out.m0] = 0;
-        if (lev[i] == l0) continue;  // reads nothing inside its group: its plain row
-        el.run(h, lev, i, l0, true);
-        const RowMap &m = el.map;
-        bool fits = (int)m.cols.size() <= kMergeMaxRow;
-        for (double v : m.vals) fits &= std::fabs(v) <= kMergeMaxAbs;
-        if (!fits) {
-          over = true;
-          return;
-        }
-        const size_t at = o.ci.size();
-        key.clear();
-        for (int p = 0; p < (int)m.cols.size(); p++) {
-          const int j = m.cols[p], l = lev[j];
-          if (l >= l0) {
-            o.ci.push_back(-2 - j);
-            o.cv.push_back(m.vals[p] / (*h.nat_diag)[j]);
-            if (!(std::fabs(o.cv.back()) <= kMergeMaxAbs)) over = true;
-          } else {
-            key.push_back(((unsigned long long)l << kKeyLevel) | ((unsigned long long)j << kKeyPos) |
-                          (unsigned)p);
-          }
-        }
-        std::sort(key.begin(), key.end());
-        for (unsigned long long q : key) {
-          const int p = (int)(q & ((1u << kKeyPos) - 1));
-          o.ci.push_back(m.cols[p]);
-          o.cv.push_back(m.vals[p]);
-        }
-        len[s - out.m0] = (int)(o.ci.size() - at);
-        out.proxy[s - out.m0] =
-            row_proxy(g, (int)key.size(), [&](int u) { return grp[(int)(key[u] >> kKeyLevel)]; });
+    int first = -1, last = -1;
+    for (int g = 0; g < G; g++) {
+      for (int l = out.gptr[g]; l < out.gptr[g + 1]; l++) grp[l] = g;
+      if (out.gptr[g + 1] - out.gptr[g] > 1) {
+        if (first < 0) first = g;
+        last = g;
       }
-      blk[b].ci.assign(o.ci.begin(), o.ci.end());
-      blk[b].cv.assign(o.cv.begin(), o.cv.end());
-      if (total.fetch_add((long long)o.ci.size()) + (long long)o.ci.size() > most)
-        over = grown = true;
     }
-  });
-  if (over) {
-    out = MergePlan();
-    return !grown;
+    out.m0 = lp[out.gptr[first] + 1];  // a group's first level reads nothing inside it
+    out.m1 = lp[out.gptr[last + 1]];
+    std::vector<std::atomic<int>> bad(G);
+    for (auto &l : bad) l = nl;
+    if (!merge_rows(h, n, lev, grp, bad, out)) {
+      out = MergePlan();
+      return false;
+    }
+    std::vector<int> gptr;
+    for (int g = 0; g < G; g++) {
+      gptr.push_back(out.gptr[g]);
+      if (bad[g] == nl) continue;
+      for (int l = bad[g]; l < (cuts < kMergeCuts ? bad[g] + 1 : out.gptr[g + 1]); l++)
+        gptr.push_back(l);
+    }
+    gptr.push_back(nl);
+    const bool done = gptr.size() == out.gptr.size();
+    out.gptr = std::move(gptr);
+    if (done) break;
   }
-  par_prefix((size_t)M, [&](size_t s) { return len[s]; }, out.rp);
-  out.ci.resize(out.rp[M]);
-  out.cv.resize(out.rp[M]);
-  par_for((size_t)B, [&](size_t b0, size_t b1) {
-    for (size_t b = b0; b < b1; b++) {
-      const int o = out.rp[b * kBlk];
-      std::copy(blk[b].ci.begin(), blk[b].ci.end(), out.ci.begin() + o);
-      std::copy(blk[b].cv.begin(), blk[b].cv.end(), out.cv.begin() + o);
-    }
-  }, 64);
   // the sweep's estimate: a handshake per group and the entries it reads
-  long long ents = h.rp[n] + (long long)out.rp[M];
+  long long ents = h.rp[n] + (long long)out.ci.size();
   for (int s = out.m0; s < out.m1; s++)
-    if (len[s - out.m0]) ents -= h.rp[s + 1] - h.rp[s];
-  out.est_us = G * kHopUs + ents * kEntryUs;
+    if (out.rp[s - out.m0 + 1] > out.rp[s - out.m0]) ents -= h.rp[s + 1] - h.rp[s];
+  out.est_us = (out.gptr.size() - 1) * kHopUs + ents * kEntryUs;
   return true;
 }
 

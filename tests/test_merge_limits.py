@@ -52,3 +52,43 @@ def test_small_factors_of_many_narrow_levels_are_merged(name, Gs):
     assert all(g <= l // 10 for g, l in zip(groups, lv)), (groups, lv)
     assert all(0 < e <= GROWTH * nnz for e in ents)
     assert rel(z, O.precond(Gs, r)) <= 1e-12
+
+
+def with_chain(rows, cols, vals, n):
+    """Given rows 0 .. n - 1, and after them a chain of 600 rows of its own."""
+    m = 600
+    rng = np.random.default_rng(3)
+    rows = np.concatenate([rows, np.arange(n + 1, n + m)])
+    cols = np.concatenate([cols, np.arange(n, n + m - 1)])
+    vals = np.concatenate([vals, -rng.uniform(0.1, 1.0, m - 1)])
+    L = sp.csc_matrix((vals, (rows, cols)), shape=(n + m, n + m))
+    return stored(L + sp.diags(np.concatenate([np.ones(n), rng.uniform(1, 2, m)])))
+
+
+def large_ratios():
+    """A chain of 20 rows whose merged coefficients pass 1e30."""
+    return with_chain(np.arange(1, 20), np.arange(19), np.full(19, -1e4), 20)
+
+
+def long_row():
+    """A row that reads 9000 others, read by one of 51 rows of its level (the
+    last: not one of those whose merged length is looked at)."""
+    k = 9000
+    side = np.arange(50)
+    rows = np.concatenate([k + 50 + side, k + 100 + side, np.full(k, k + 150), [k + 151]])
+    cols = np.concatenate([k + side, k + 50 + side, np.arange(k), [k + 150]])
+    return with_chain(rows, cols, np.full(rows.size, -1e-3), k + 152)
+
+
+@pytest.mark.parametrize("second", [large_ratios, long_row])
+def test_a_row_that_cannot_be_merged_leaves_its_group_alone(second):
+    """Not the whole sweep: the other chain is merged."""
+    Gs = second()
+    n = len(Gs[0]) - 1
+    r = np.random.default_rng(8).uniform(0.1, 1, n)
+    z, groups, ents, est = merge_apply_host(Gs, r)
+    lv = levels(Gs)
+    assert groups[0] < lv[0] // 2 and ents[0] > 0, (groups, lv, ents)
+    # rounding of sums of one sign in either order, relative to each value
+    zo = O.precond(Gs, r)
+    assert np.max(np.abs(z - zo) / np.abs(zo)) <= 1e-11

@@ -201,11 +201,11 @@ bool merge_signs(const HostSweep &h, size_t n) {
   return ok;
 }
 
-// Groups of consecutive levels [a, b): a group grows by the next level while
-// that level's rows, merged, stay within kMergeLen entries on average and the
-// entries that merging adds to the level cost less than kMergeCapUs of the
-// handshake they save.  Merged lengths come from a sample of the level's
-// rows.  Neighbouring groups are about as deep as each other, so the search
+// Groups of consecutive levels [a, b): a group grows by its next levels (an
+// eighth of its depth at a time) while their rows, merged, stay within lim.len
+// entries on average and the entries that merging adds to a level cost less
+// than lim.cap_us.  Merged lengths come from a sample of the rows of the last
+// level.  Neighbouring groups are about as deep as each other, so the search
 // starts at the depth of the last one and goes up or down from there.
 constexpr int kMergeSample = 6;
 
@@ -213,7 +213,8 @@ void plan_groups(const HostSweep &h, const IntVec &lev, int a, int b, const Merg
                  std::vector<int> &gptr) {
   const std::vector<int> &lp = h.level_ptr;
   RowElim el(h.nat_rp.size() - 1);
-  auto mean_merged = [&](int m, int l0, double &merged, double &plain) {
+  double merged = 0.0, plain = 0.0;  // mean entries of the rows that fits() looked at last
+  auto mean_merged = [&](int m, int l0) {
     const int w = lp[m + 1] - lp[m], k = std::min(w, kMergeSample);
     merged = plain = 0.0;
     for (int t = 0; t < k; t++) {
@@ -224,19 +225,30 @@ void plan_groups(const HostSweep &h, const IntVec &lev, int a, int b, const Merg
     merged /= k;
     plain /= k;
   };
-  // whether the group [l, e) may hold its last levels (an eighth of them)
+  auto widest = [&](int l0, int l1) {
+    int w = 0;
+    for (int q = l0; q < l1; q++) w = std::max(w, lp[q + 1] - lp[q]);
+    return (double)w;
+  };
+  // whether the group [l, e) may hold its last levels (a ninth of them)
   auto fits = [&](int l, int e) {
-    double merged, plain, worst = 0.0;
-    mean_merged(e - 1, l, merged, plain);
-    for (int q = e - std::max(1, (e - l) / 9); q < e; q++)
-      worst = std::max(worst, (double)(lp[q + 1] - lp[q]));
-    return merged <= lim.len && (merged - plain) * worst * kEntryUs <= lim.cap_us;
+    mean_merged(e - 1, l);
+    return merged <= lim.len &&
+           (merged - plain) * widest(e - std::max(1, (e - l) / 9), e) * kEntryUs <= lim.cap_us;
   };
   int depth = 1;
   for (int l = a; l < b;) {
     const int guess = std::min(b, l + depth);
     int e = guess;
     while (e - l > 1 && !fits(l, e)) e = std::max(l + 1, e - std::max(1, (e - l) / 8));
+    // the levels below the last: their rows are no longer than the last one's,
+    // but a level may be wider
+    const double longest = merged;
+    for (int q = l + 1; q < e;) {
+      const int m = std::min(e, q + std::max(1, (q - l) / 8));
+      if (m < e && longest * widest(q, m) * kEntryUs > lim.cap_us && !fits(l, m)) e = q;
+      q = m;
+    }
     while (e >= guess && e < b) {
       const int m = std::min(b, e + std::max(1, (e - l) / 8));
       if (!fits(l, m)) break;

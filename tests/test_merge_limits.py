@@ -92,3 +92,33 @@ def test_a_row_that_cannot_be_merged_leaves_its_group_alone(second):
     # rounding of sums of one sign in either order, relative to each value
     zo = O.precond(Gs, r)
     assert np.max(np.abs(z - zo) / np.abs(zo)) <= 1e-11
+
+
+def chain_with_wide_levels(n, wide, w):
+    """A chain of n rows in which every level of `wide` also holds w rows that
+    read the chain's row before."""
+    rows, cols = [np.arange(1, n)], [np.arange(n - 1)]
+    k = n
+    for l in wide:
+        rows.append(np.arange(k, k + w))
+        cols.append(np.full(w, l - 1))
+        k += w
+    rows, cols = np.concatenate(rows), np.concatenate(cols)
+    rng = np.random.default_rng(5)
+    L = sp.csc_matrix((-rng.uniform(0.1, 1.0, rows.size), (rows, cols)), shape=(k, k))
+    return stored(L + sp.diags(rng.uniform(1, 2, k)))
+
+
+def test_a_wide_level_inside_a_group_is_looked_at():
+    """A level of w rows is merged only while the entries this adds cost less
+    than 0.2 us at 5 ps each, wherever in a group's depth it lies: the wide
+    levels at 100 and 150 hold 3000 rows, so none of their rows may have more
+    than 14 entries (0.2 / 5e-6 / 3000, and the one it reads)."""
+    n, w = 400, 3000
+    Gs = chain_with_wide_levels(n, [100, 150], w)
+    r = np.random.default_rng(8).uniform(-1, 1, n + 2 * w)
+    z, groups, ents, est = merge_apply_host(Gs, r)
+    assert rel(z, O.precond(Gs, r)) <= 1e-12
+    assert groups[0] < levels(Gs)[0] // 10
+    # the chain's own rows: at most one triangle of n / 2 each way
+    assert ents[0] <= n * n // 2 + 2 * w * 14, (groups, ents)

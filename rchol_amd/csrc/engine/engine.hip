@@ -1860,7 +1860,7 @@ int rchol_amd_upload_G(rchol_amd_ctx *c, size_t n, const size_t *colPtr, const s
   } join{planner};
   if (c->merge_levels && c->chunk_mode != 1) {
     auto plan = [&]() {
-      const MergeLimits lim = merge_limits(is_deep(n, nlf, nlb), n, nnz);
+      const MergeLimits lim = merge_limits(is_deep(n, nlf, nlb), n, nnz, precision);
       for (int k = 0; k < 2; k++) try {
           plan_merge(k ? hb : hf, n, lim, mplan[k]);
         } catch (const std::exception &) {  // no memory or threads for it: the plain levels
@@ -2689,7 +2689,7 @@ int rchol_amd_merge_apply_host(size_t n, const size_t *colPtr, const size_t *row
   int rc = analyze_factor(n, colPtr, rowIdx, val, hf, hb, nlf, nlb);
   if (rc) return rc;
   MergePlan pf, pb;
-  const MergeLimits lim = merge_limits(is_deep(n, nlf, nlb), n, colPtr[n]);
+  const MergeLimits lim = merge_limits(is_deep(n, nlf, nlb), n, colPtr[n], RCHOL_AMD_FP64);
   plan_merge(hf, n, lim, pf);
   plan_merge(hb, n, lim, pb);
   std::vector<double> y(n);

@@ -33,10 +33,12 @@
 constexpr double kHopUs = RCHOL_AMD_MERGE_HOP;
 constexpr double kEntryUs = RCHOL_AMD_MERGE_PS * 1e-6;
 // How far a level is merged: microseconds of entries that merging may add to
-// it, mean entries of its merged rows; most levels of a sweep that is merged.
+// it, mean entries of its merged rows; most levels of a sweep that is merged;
+// largest coefficient of a merged row, in pivots of the row.
 struct MergeLimits {
   double cap_us, len;
   int levels;
+  double ratio;
 };
 constexpr int kMergeMaxLevels = 1 << 20;  // (fits the sort key of a merged entry)
 #ifndef RCHOL_AMD_MERGE_CAP
@@ -60,11 +62,18 @@ constexpr int kMergeMaxLevels = 1 << 20;  // (fits the sort key of a merged entr
 #endif
 constexpr double kDeepGrowth = 96.0;
 constexpr int kDeepMaxLevels = 16384;
-MergeLimits merge_limits(bool deep, size_t n, size_t nnz) {
-  if (!deep) return {RCHOL_AMD_MERGE_CAP, RCHOL_AMD_MERGE_LEN, kMergeMaxLevels};
+// Largest coefficient of a merged row in pivots of the row.  Beyond the
+// reciprocal of the unit roundoff a term x_k c / d says nothing of a result of
+// ordinary size: the row's terms cancel.  The substitution cancels them one
+// dependency at a time; merged, each is formed whole, and in FP32 c x_k may
+// pass the largest number.
+constexpr double kMergeRatio32 = 1e8;
+MergeLimits merge_limits(bool deep, size_t n, size_t nnz, int precision) {
+  const double ratio = precision == RCHOL_AMD_FP32 ? kMergeRatio32 : HUGE_VAL;
+  if (!deep) return {RCHOL_AMD_MERGE_CAP, RCHOL_AMD_MERGE_LEN, kMergeMaxLevels, ratio};
   return {RCHOL_AMD_MERGE_DEEP_CAP,
           std::min<double>(RCHOL_AMD_MERGE_DEEP_LEN, kDeepGrowth * (double)nnz / (double)n),
-          kDeepMaxLevels};
+          kDeepMaxLevels, ratio};
 }
 
 struct MergePlan {
@@ -267,7 +276,7 @@ void plan_groups(const HostSweep &h, const IntVec &lev, int a, int b, const Merg
 // elimination meets them: sweeps 4 to 18% slower).  bad[g]: lowered to the
 // lowest level of group g with a row that cannot be merged (which is left
 // out).  False: more merged entries than kMergeMaxGrowth allows.
-bool merge_rows(const HostSweep &h, size_t n, const IntVec &lev, const IntVec &grp,
+bool merge_rows(const HostSweep &h, size_t n, const IntVec &lev, const IntVec &grp, double ratio,
                 std::vector<std::atomic<int>> &bad, MergePlan &out) {
   const int M = out.m1 - out.m0;
   constexpr int kBlk = 64;
@@ -298,7 +307,8 @@ bool merge_rows(const HostSweep &h, size_t n, const IntVec &lev, const IntVec &g
         el.run(h, lev, i, l0, true);
         const RowMap &m = el.map;
         bool fits = (int)m.cols.size() <= kMergeMaxRow;
-        for (double v : m.vals) fits &= std::fabs(v) <= kMergeMaxAbs;
+        const double most_v = std::min(kMergeMaxAbs, ratio * std::fabs((*h.nat_diag)[i]));
+        for (double v : m.vals) fits &= std::fabs(v) <= most_v;
         for (int p = 0; p < (int)m.cols.size(); p++)
           if (lev[m.cols[p]] >= l0)
             fits &= std::fabs(m.vals[p] / (*h.nat_diag)[m.cols[p]]) <= kMergeMaxAbs;
@@ -350,7 +360,7 @@ bool merge_rows(const HostSweep &h, size_t n, const IntVec &lev, const IntVec &g
 
 // The groups and merged rows of one sweep within the limits (empty when no two
 // levels are worth merging).  A group with rows that cannot be merged (longer
-// than kMergeMaxRow, a coefficient beyond kMergeMaxAbs) is cut where the lowest
+// than kMergeMaxRow, a coefficient too large) is cut where the lowest
 // of them stands, up to kMergeCuts times; what is left of it then stays as its
 // plain levels.  False: more merged entries than kMergeMaxGrowth allows.
 bool plan_within(const HostSweep &h, size_t n, const IntVec &lev, const MergeLimits &lim,
@@ -402,7 +412,7 @@ bool plan_within(const HostSweep &h, size_t n, const IntVec &lev, const MergeLim
     out.m1 = lp[out.gptr[last + 1]];
     std::vector<std::atomic<int>> bad(G);
     for (auto &l : bad) l = nl;
-    if (!merge_rows(h, n, lev, grp, bad, out)) {
+    if (!merge_rows(h, n, lev, grp, lim.ratio, bad, out)) {
       out = MergePlan();
       return false;
     }

@@ -463,6 +463,7 @@ struct rchol_amd_ctx {
   int merge_levels = 1;     // RCHOL_AMD_OPT_MERGE
   bool chunk_auto = false;  // the upload's own choice (chunk_mode -1)
   double chunk_est_us = 0.0;  // both sweeps in chunks, planned with the last factor
+  bool chunks_linked = false;  // some chunk reads another
   bool use_chunks = false;  // single-RHS sweeps run k_sptrsv_chunk
   int lds_max = 0;          // LDS bytes a workgroup may allocate
   int chunk_grid = 0;       // workgroups of the chunked sweeps
@@ -1809,6 +1810,7 @@ int setup_chunks(rchol_amd_ctx *c, size_t n, HostSweep &hf, HostSweep &hb, int n
   plan_chunks(hf, (int)n, bnd, false, pf);
   plan_chunks(hb, (int)n, bnd, true, pb);
   c->chunk_est_us = pf.est_us + pb.est_us;
+  c->chunks_linked = !pf.dep.empty() || !pb.dep.empty();
   c->chunk_auto = c->chunk_est_us < (nlf + nlb) * kLevelUs;
   if (c->chunk_mode == -1 && !c->chunk_auto) return RCHOL_AMD_OK;
   int rc = upload_chunks(c->fwd.ch, pf, precision);
@@ -1823,6 +1825,25 @@ int setup_chunks(rchol_amd_ctx *c, size_t n, HostSweep &hf, HostSweep &hb, int n
   }
   c->use_chunks = true;
   return RCHOL_AMD_OK;
+}
+
+// Whether the merged levels of a deep factor take the place of its chunks: by
+// the estimates, the chunks' raised by half where chunks read each other (the
+// hand-over from chunk to chunk takes longer than estimated).
+//
+// Both forms of 41 factors (natural and static orders of 2D and 3D grids from
+// 64^2 to 1000x600 and 14^3 to 88^3, chains, and stacks of 4 to 2000 of them;
+// FP64 / FP32, merged over chunked time of one application) against merged
+// over chunked estimate:
+//   chunks that read each other: 0.15 ... 0.56 at estimates 0.1 ... 0.55 (0.74
+//   at most), 0.62 / 0.67 at 1.01 (static 72^3), 0.60 / 0.63 at 1.24 (88^3),
+//   0.72 / 0.76 at 1.41 (160x160x20); 1.56 / 1.67 at 1.96, 1.87 / 1.76 at 2.78
+//   (stacks of 32 natural 16^3 and 16 static 32^3)
+//   chunks that do not: 0.61 / 0.71 at 0.93 (256 chains of 2000 rows), 1.24 /
+//   1.50 at 1.01 (32 natural 64x64 grids), 2.24 / 2.58 at 2.69 (128 of them)
+bool merged_wins(const rchol_amd_ctx *c, const MergePlan &f, const MergePlan &b) {
+  return f.any() && b.any() &&
+         f.est_us + b.est_us < (c->chunks_linked ? 1.5 : 1.0) * c->chunk_est_us;
 }
 
 }  // namespace
@@ -1925,13 +1946,7 @@ int rchol_amd_upload_G(rchol_amd_ctx *c, size_t n, const size_t *colPtr, const s
   if (!rc) rc = up(c->bwd, hb);
   if (!rc) rc = setup_chunks(c, n, hf, hb, nlf, nlb, precision);
   if (planner.joinable()) planner.join();
-  // A deep factor has both plans: the merged levels when they are estimated
-  // faster, the chunks' estimate raised to what they take (estimated / taken,
-  // both sweeps, ms: merged 0.16 / 0.25 at 24^3 natural, 0.55 / 1.10 at static
-  // 40^3, 1.98 / 2.12 at 64^3, 2.86 / 2.96 at 72^3; chunks 0.49 / 0.58,
-  // 0.92 / 1.46, 2.01 / 3.44 and 2.64 / 4.87)
-  if (c->use_chunks && c->chunk_mode == -1 && mplan[0].any() && mplan[1].any() &&
-      mplan[0].est_us + mplan[1].est_us < 1.5 * c->chunk_est_us) {
+  if (c->use_chunks && c->chunk_mode == -1 && merged_wins(c, mplan[0], mplan[1])) {
     c->chunk_auto = false;
     c->use_chunks = false;
   }

@@ -113,10 +113,11 @@ struct DevBuf {
     p = nullptr;
     n = 0;
   }
-  hipError_t alloc(size_t count) {
+  hipError_t alloc(size_t count) {  // failed: empty
     reset();
-    n = count;
-    return hipMalloc((void **)&p, std::max<size_t>(count, 1) * sizeof(T));
+    const hipError_t e = hipMalloc((void **)&p, std::max<size_t>(count, 1) * sizeof(T));
+    if (e == hipSuccess) n = count; else p = nullptr;
+    return e;
   }
   hipError_t upload(const T *h, size_t count) {
     hipError_t e = alloc(count);
@@ -1921,38 +1922,57 @@ int rchol_amd_upload_G(rchol_amd_ctx *c, size_t n, const size_t *colPtr, const s
     return precision == RCHOL_AMD_FP32 ? gather_slots<float>(c, sw, h, sw.cv32, sw.diag32)
                                        : gather_slots<double>(c, sw, h, sw.cv64, sw.diag64);
   };
-  auto up_merged = [&](Sweep &sw, MergePlan &mp) -> int {
-    sw.m0 = mp.m0;
-    sw.m1 = mp.m1;
-    sw.gptr_h = std::move(mp.gptr);
-    sw.mrp_h.assign(mp.rp.begin(), mp.rp.end());
-    sw.mproxy_h.resize(mp.proxy.size());
-    for (size_t k = 0; k < mp.proxy.size(); k++)
-      sw.mproxy_h[k] = mp.proxy[k] ? mp.ci[mp.rp[k + 1] - 1 - mp.proxy[k]] : -1;
+  auto drop_merged = [](Sweep &sw) {
+    sw.m0 = sw.m1 = 0;
+    sw.gptr_h.clear();
+    sw.mrp_h.clear();
+    sw.mproxy_h.clear();
     sw.mrp.reset();
     sw.mci.reset();
     sw.mcv64.reset();
     sw.mcv32.reset();
-    if (sw.m1 == sw.m0) return RCHOL_AMD_OK;
+  };
+  auto up_merged = [&](Sweep &sw, MergePlan &mp) -> int {
+    if (!mp.any()) return RCHOL_AMD_OK;
     HIP_TRY(sw.mrp.upload(mp.rp.data(), mp.rp.size()));
     HIP_TRY(sw.mci.upload(mp.ci.data(), mp.ci.size()));
     if (precision == RCHOL_AMD_FP32)
       HIP_TRY(upload_as(sw.mcv32, mp.cv));
     else
       HIP_TRY(upload_as(sw.mcv64, mp.cv));
+    sw.mrp_h.assign(mp.rp.begin(), mp.rp.end());
+    sw.mproxy_h.resize(mp.proxy.size());
+    for (size_t k = 0; k < mp.proxy.size(); k++)
+      sw.mproxy_h[k] = mp.proxy[k] ? mp.ci[mp.rp[k + 1] - 1 - mp.proxy[k]] : -1;
+    sw.gptr_h = std::move(mp.gptr);
+    sw.m0 = mp.m0;
+    sw.m1 = mp.m1;
     return RCHOL_AMD_OK;
   };
   int rc = up(c->fwd, hf);
   if (!rc) rc = up(c->bwd, hb);
   if (!rc) rc = setup_chunks(c, n, hf, hb, nlf, nlb, precision);
   if (planner.joinable()) planner.join();
-  if (c->use_chunks && c->chunk_mode == -1 && merged_wins(c, mplan[0], mplan[1])) {
+  drop_merged(c->fwd);
+  drop_merged(c->bwd);
+  if (rc) return rc;
+  // the merged rows only make the sweeps faster: without the memory for them
+  // the plain levels, or the chunks, run
+  const bool merged_win = c->use_chunks && c->chunk_mode == -1 && merged_wins(c, mplan[0], mplan[1]);
+  bool merged = false;
+  try {
+    merged = !up_merged(c->fwd, mplan[0]) && !up_merged(c->bwd, mplan[1]);
+  } catch (const std::bad_alloc &) {
+  }
+  if (!merged) {
+    (void)hipGetLastError();
+    drop_merged(c->fwd);
+    drop_merged(c->bwd);
+  }
+  if (merged && merged_win) {
     c->chunk_auto = false;
     c->use_chunks = false;
   }
-  if (!rc) rc = up_merged(c->fwd, mplan[0]);
-  if (!rc) rc = up_merged(c->bwd, mplan[1]);
-  if (rc) return rc;
   c->nG = n;
   c->nnzG = nnz;
   c->gprec = precision;

@@ -97,8 +97,10 @@ typedef struct rchol_amd_stats {
   /* Host wall time of the last uploads: [0] rchol_amd_upload_A (checks,
    * index narrowing, copies), and of rchol_amd_upload_G [1] the factor
    * analysis (validation, levels, slot-ordered CSR of both sweeps), [2] the
-   * sweep schedule (task cut, per-wave lists), [3] the FP32 conversion (FP32
-   * factor) and the copies to the device. */
+   * sweep schedule (the chunked plan with its copies, the wait for the merge
+   * plan, which is made beside [3] and the chunked one, task cut, per-wave
+   * lists), [3] the FP32 conversion (FP32 factor) and the copies of the plain
+   * and the merged rows to the device. */
   double setup_ms[4];
   /* 1 when the single-right-hand-side sweeps run chunked; chunks and rounds
    * of internal entries of [0] the forward and [1] the backward plan (0: no

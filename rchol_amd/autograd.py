@@ -17,7 +17,15 @@ import numpy as np
 import torch
 
 from . import factor as F
-from .solver import FP32, FP64, Solver
+from .solver import FP32, FP64, OPT_MERGE, Solver
+
+
+# From this reuse of a cached factor on its sweeps run on merged levels.  Their
+# plan is paid back by 3 to 5 solves (32^3 13 ms for 3.1 ms a solve, 64^3 23 for
+# 4.6, 97x61x83 23 for 5.5, 128^3 24 for 7.6; made later it costs the plain
+# upload once more, 6 to 97 ms), and a training step whose weights change has
+# two for each factor.
+MERGE_AT_REUSE = 3
 
 
 class GridLaplacian:
@@ -45,6 +53,8 @@ class GridLaplacian:
         self._key = None
         self._solver = None
         self._w = None  # device copy of the weights the cached factor belongs to
+        self._factor = None  # its host arrays, until it is uploaded with merged levels
+        self._reuses = 0
         self.last = {}
 
     def matrix(self, w):
@@ -56,25 +66,48 @@ class GridLaplacian:
         The cache holds only the latest solver.  A replaced solver is not
         closed here: a forward pass whose backward is still pending keeps
         its own solver alive through its autograd context, and the context
-        is freed (closing the solver) once that backward has run."""
+        is freed (closing the solver) once that backward has run.
+
+        A new factor runs on its plain levels, the shorter upload; one that is
+        asked for again MERGE_AT_REUSE times is uploaded to the same solver
+        with merged levels."""
         w = np.ascontiguousarray(w, dtype=np.float64)
         key = hashlib.blake2b(w.tobytes(), digest_size=32).digest()
-        if key != self._key:
-            A = self.matrix(w)
-            Gs, po, _ = F.factor(A, self._perm, self._blocks, self.order, self.seed)
-            Ap = F.permute(A, po)
-            s = Solver(Ap, Gs, self.precision, device=self.device)
-            s.set_perm(po)
-            self._solver = s
-            self._key = key
-        return self._solver
+        if key == self._key:
+            return self._reused()
+        self._factor = None  # not beside the new one
+        A = self.matrix(w)
+        Gs, po, _ = F.factor(A, self._perm, self._blocks, self.order, self.seed)
+        s = Solver(F.permute(A, po), device=self.device)
+        s.set_option(OPT_MERGE, 0)
+        s.upload_G(Gs, self.precision)
+        s.set_perm(po)
+        self._solver = s
+        self._key = key
+        self._factor = Gs
+        self._reuses = 0
+        return s
+
+    def _reused(self):
+        """The cached solver, asked for once more."""
+        s = self._solver
+        self._reuses += 1
+        if self._reuses >= MERGE_AT_REUSE and self._factor is not None:
+            Gs, self._factor = self._factor, None
+            s.set_option(OPT_MERGE, 1)
+            try:
+                s.upload_G(Gs, self.precision)
+            except RuntimeError:  # what was there before
+                s.set_option(OPT_MERGE, 0)
+                s.upload_G(Gs, self.precision)
+        return s
 
     def solver_for(self, w):
         """Solver for the weights of a device tensor: the cached factor is
         reused when w equals (on the device) the weights it was built for."""
         if self._solver is not None and self._w is not None and self._w.shape == w.shape \
                 and torch.equal(self._w, w):
-            return self._solver
+            return self._reused()
         s = self.solver(w.detach().cpu().numpy())
         self._w = w.detach().clone()
         return s

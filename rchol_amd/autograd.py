@@ -84,6 +84,7 @@ class GridLaplacian:
         s.set_perm(po)
         self._solver = s
         self._key = key
+        self._w = None  # solver_for sets it
         self._factor = Gs
         self._reuses = 0
         return s

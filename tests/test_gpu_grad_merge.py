@@ -58,3 +58,22 @@ def test_a_factor_that_is_kept_is_merged(precision):
         assert prob._factor is None
         for g in grads[1:]:  # both solves to 1e-12
             assert float((g - grads[0]).norm() / grads[0].norm()) <= 1e-9
+
+
+def test_a_solver_of_other_weights_is_not_reused():
+    """solver() between two passes on the same tensor: the second pass has its
+    own weights' factor, not the cache's latest."""
+    import torch
+    from rchol_amd import autograd as AG
+    if rchol_amd.device_count() < 1:
+        pytest.skip("no HIP device")
+    prob = AG.GridLaplacian(*DIMS, leaves=4, precision=rchol_amd.FP64, tol=1e-12)
+    rng = np.random.default_rng(5)
+    w, other = (rng.uniform(0.5, 2.0, prob.m) for _ in range(2))
+    wt = torch.as_tensor(w, device="cuda")
+    b = torch.as_tensor(rng.uniform(-1.0, 1.0, prob.n), device="cuda")
+    print("case other weights", flush=True)
+    x = AG.solve(wt, b, prob)
+    prob.solver(10.0 * other)
+    y = AG.solve(wt, b, prob)
+    assert float((x - y).norm() / x.norm()) <= 1e-9  # both to 1e-12

@@ -61,8 +61,8 @@ typedef struct rchol_amd_ctx rchol_amd_ctx;
                                          orders) instead of level by level.  -1 (default):
                                          planned at upload_G when the factor has many narrow
                                          levels, used when its estimate beats the level
-                                         schedule, merged or not; 0: never; 1: always (planned at the next
-                                         upload_G; set before it) */
+                                         schedule, merged or not; 0: never; 1: always
+                                         (planned at the next upload_G; set before it) */
 #define RCHOL_AMD_OPT_WAIT_TICKS 11   /* bound of every dependency / residency wait, in
                                          ticks of the 100 MHz wall clock, for the GPU of
                                          this context (every context on it); 0 restores
@@ -72,8 +72,11 @@ typedef struct rchol_amd_ctx rchol_amd_ctx;
 #define RCHOL_AMD_OPT_MERGE 12        /* 1 (default): the next upload_G merges consecutive narrow
                                          levels of the sweeps (one to eight columns) into
                                          groups of one handshake each, where the factor's
-                                         signs allow it; 0: it does not (a shorter upload, for
-                                         a factor that is used once) */
+                                         signs allow it and the device has room for the
+                                         merged rows; 0: it does not (a shorter upload, for a
+                                         factor of fewer solves than earn the plan back:
+                                         3 to 5 for independent-set orders, 6 to 10 for deep
+                                         ones) */
 
 /* Counters filled by rchol_amd_get_stats. */
 typedef struct rchol_amd_stats {

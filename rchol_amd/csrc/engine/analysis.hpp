@@ -293,12 +293,10 @@ void build_slots(const IntVec &lev, int nlev, HostSweep &hs) {
 }
 
 // Inside every row, entries ordered by the level of the row they read,
-// latest last, ties by column, then by value.  Single-column sweeps read a
-// row from its end, so the lane that polls for a wave watches the value
-// produced last and, when it lands, the rest of the row is usually there
-// too.  Multi-column sweeps read from the start, several rounds per row: the
-// rounds over long-finished entries run while the latest are still in
-// flight.  The key fixes the order whatever order the entries arrive in.
+// latest last, ties by column, then by value.  The sweeps cut a row into rounds
+// from its end and run the oldest round first: the lane that polls for a wave
+// watches the value produced last, and the rounds before run while it is still
+// in flight.  The key fixes the order whatever order the entries arrive in.
 struct LevelEnt {
   unsigned long long key;  // level << 32 | column
   double v;

@@ -85,10 +85,7 @@ __device__ __forceinline__ T ld_stream(const T *p) {
   return *p;
 #endif
 }
-// The same as a choice of the kernel.  The single-column sweeps load plainly
-// at every size (both sweeps, non-temporal -> plain: 97x61x83 FP32 0.33 ->
-// 0.31 ms, 128^3 FP32 0.73 -> 0.70 ms, 256^3 2.60 -> 2.55 ms: their matrices
-// come back from the Infinity Cache as far as they fit it).
+// The same as a choice of the kernel (the SpMV's stream form).
 template <bool NT, typename T>
 __device__ __forceinline__ T ld_once(const T *p) {
   if constexpr (NT) return __builtin_nontemporal_load(p);
@@ -111,7 +108,6 @@ __device__ long long g_wait_ticks = kWaitTicks;
 #define RCHOL_AMD_POLL_CAP 8
 #endif
 constexpr int kPollCap = RCHOL_AMD_POLL_CAP;
-
 
 // The bound and back-off of one wait.
 struct Poll {

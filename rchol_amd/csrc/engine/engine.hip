@@ -552,10 +552,6 @@ struct rchol_amd_ctx {
     if (g > 8) g = (g + 7) / 8 * 8;  // whole XCD rounds for the row walk of the stream form
     return (int)g;
   }
-  // A larger than half the Infinity Cache streams past the caches in the SpMV,
-  // a smaller one is left in them for the next iteration (stream form, plain
-  // / non-temporal: 48 ... 100^3 and 2D stacks 5 to 10% faster plain, 97x61x83
-  // 26.4 / 28.7 us; 128^3 77 / 75 us, 160^3 139 / 132 us)
   // Grid of the K-column SpMV (kCols columns per lane): at least two row steps
   // per wave, since every workgroup adds to the reduction that ends the kernel
   // (24^3, K = 32: 40 us with one step, 28 with two, 29 with eight), whole XCD
@@ -566,6 +562,10 @@ struct rchol_amd_ctx {
                                                     (size_t)ncu * kSpmvMrBlocksPerCu));
     return (int)(g > 8 ? (g + 7) / 8 * 8 : g);
   }
+  // A larger than half the Infinity Cache streams past the caches in the SpMV,
+  // a smaller one is left in them for the next iteration (stream form, plain
+  // / non-temporal: 48 ... 100^3 and 2D stacks 5 to 10% faster plain, 97x61x83
+  // 26.4 / 28.7 us; 128^3 77 / 75 us, 160^3 139 / 132 us)
   bool spmv_nt() const { return nnzA * 12 > (128u << 20); }
   int ensure_work();
   int size_trsv_grid();
@@ -630,9 +630,9 @@ void launch_one_sweep(rchol_amd_ctx *c, const Sweep &sw, const VT *cv, const VT 
                        sw.ci.p, cv, dg, rhs, x, aux, dotv, sc, stop, 0);
   if (sw.mid_ntasks > 0 || (FUSE == 2 && !tail))
     hipLaunchKernelGGL((k_sptrsv<VT, XT, BT, FUSE>), dim3(c->trsv_grid), dim3(kBlock), 0,
-                       c->stream, sw.wave_ptr.p, sw.wt.p,
-                       sw.slot_row.p, sw.rp.p, sw.ci.p, cv, mrp, (const int *)sw.mci.p, mcv, dg, rhs, x, aux, dotv, c->partials.p, sc, stop, tail ? 1 : 0,
-                       c->coherent_gather);
+                       c->stream, sw.wave_ptr.p, sw.wt.p, sw.slot_row.p, sw.rp.p, sw.ci.p, cv, mrp,
+                       (const int *)sw.mci.p, mcv, dg, rhs, x, aux, dotv, c->partials.p, sc, stop,
+                       tail ? 1 : 0, c->coherent_gather);
   if (tail)
     hipLaunchKernelGGL((k_sptrsv_serial<VT, XT, BT, FUSE>), dim3(1), dim3(1024), 0, c->stream,
                        sw.tail_begin, sw.nlevels, sw.level_ptr.p, sw.level_lg.p, sw.slot_row.p,
@@ -1070,27 +1070,39 @@ void rchol_amd_ctx::launch_sweeps_mr(const double *rhs, bool with_dot, const int
   const int *mrpf = fwd.mrp.p ? fwd.mrp.p - fwd.m0 : nullptr;
   const int *mrpb = bwd.mrp.p ? bwd.mrp.p - bwd.m0 : nullptr;
   if (gprec == RCHOL_AMD_FP32) {
-    hipLaunchKernelGGL((k_sptrsv_mr<float, float, double, K, 1>), g, blk, 0, stream, wpf, wtf, fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv32.p, mrpf, fwd.mci.p, fwd.mcv32.p, fwd.diag32.p, rhs,
+    hipLaunchKernelGGL((k_sptrsv_mr<float, float, double, K, 1>), g, blk, 0, stream, wpf, wtf,
+                       fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv32.p, mrpf,
+                       fwd.mci.p, fwd.mcv32.p, fwd.diag32.p, rhs,
                        batch.y32.p, batch.z32.p, nullptr, nullptr, batch.bs, stop);
     if (ev) (void)hipEventRecord(ev[1], stream);
     if (with_dot)
-      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 2>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, mrpb, bwd.mci.p, bwd.mcv32.p, bwd.diag32.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 2>), g, blk, 0, stream, wpb, wtb,
+                         bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, mrpb,
+                         bwd.mci.p, bwd.mcv32.p, bwd.diag32.p,
                          (const float *)batch.y32.p, batch.z32.p, (float *)nullptr,
                          (const double *)batch.r.p, batch.partials.p, batch.bs, stop);
     else
-      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 0>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, mrpb, bwd.mci.p, bwd.mcv32.p, bwd.diag32.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<float, float, float, K, 0>), g, blk, 0, stream, wpb, wtb,
+                         bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv32.p, mrpb,
+                         bwd.mci.p, bwd.mcv32.p, bwd.diag32.p,
                          (const float *)batch.y32.p, batch.z32.p, (float *)nullptr, nullptr,
                          nullptr, batch.bs, stop);
   } else {
-    hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 1>), g, blk, 0, stream, wpf, wtf, fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv64.p, mrpf, fwd.mci.p, fwd.mcv64.p, fwd.diag64.p, rhs,
+    hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 1>), g, blk, 0, stream, wpf, wtf,
+                       fwd.slot_row.p, fwd.rp.p, fwd.ci.p, fwd.cv64.p, mrpf,
+                       fwd.mci.p, fwd.mcv64.p, fwd.diag64.p, rhs,
                        batch.y64.p, batch.z64.p, nullptr, nullptr, batch.bs, stop);
     if (ev) (void)hipEventRecord(ev[1], stream);
     if (with_dot)
-      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 2>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, mrpb, bwd.mci.p, bwd.mcv64.p, bwd.diag64.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 2>), g, blk, 0, stream, wpb, wtb,
+                         bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, mrpb,
+                         bwd.mci.p, bwd.mcv64.p, bwd.diag64.p,
                          (const double *)batch.y64.p, batch.z64.p, (double *)nullptr,
                          (const double *)batch.r.p, batch.partials.p, batch.bs, stop);
     else
-      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 0>), g, blk, 0, stream, wpb, wtb, bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, mrpb, bwd.mci.p, bwd.mcv64.p, bwd.diag64.p,
+      hipLaunchKernelGGL((k_sptrsv_mr<double, double, double, K, 0>), g, blk, 0, stream, wpb, wtb,
+                         bwd.slot_row.p, bwd.rp.p, bwd.ci.p, bwd.cv64.p, mrpb,
+                         bwd.mci.p, bwd.mcv64.p, bwd.diag64.p,
                          (const double *)batch.y64.p, batch.z64.p, (double *)nullptr, nullptr,
                          nullptr, batch.bs, stop);
   }
@@ -1210,8 +1222,9 @@ int rchol_amd_ctx::pcg_batch(const double *d_b, int ncols, double tol, int maxit
   }
   if (batch.hbs->err)
     return stall(batch.hbs->err);
-  hipLaunchKernelGGL((k_spmv_res_mr<K>), dim3(spmv_mr_grid(K)), dim3(kBlock), 0, stream, (int)n, arp.p, aci.p,
-                     av.p, (const double *)batch.x.p, d_b, batch.res.p, batch.partials.p, batch.bs);
+  hipLaunchKernelGGL((k_spmv_res_mr<K>), dim3(spmv_mr_grid(K)), dim3(kBlock), 0, stream, (int)n,
+                     arp.p, aci.p, av.p, (const double *)batch.x.p, d_b, batch.res.p,
+                     batch.partials.p, batch.bs);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(ev1, stream));
   HIP_TRY(hipMemcpyAsync(batch.hbs, batch.bs, sizeof(BatchScalars), hipMemcpyDeviceToHost, stream));
@@ -1439,7 +1452,11 @@ int rchol_amd_ctx::pcg_segments(const double *d_b, double tol, int maxit, double
   if (hsc->err)
     return stall(hsc->err);
   switch (spmv_lanes) {
-    case 0: hipLaunchKernelGGL(spmv_nt() ? k_spmv_res_seg_s<true> : k_spmv_res_seg_s<false>, dim3(segs.nblocks), dim3(kBlock), 0, stream, lay, arp.p, aci.p, av.p, (const double *)x.p, d_b, tmp64a.p, partials.p, segs.ss); break;
+    case 0:
+      hipLaunchKernelGGL(spmv_nt() ? k_spmv_res_seg_s<true> : k_spmv_res_seg_s<false>,
+                         dim3(segs.nblocks), dim3(kBlock), 0, stream, lay, arp.p, aci.p, av.p,
+                         (const double *)x.p, d_b, tmp64a.p, partials.p, segs.ss);
+      break;
     case 4: hipLaunchKernelGGL((k_spmv_res_seg<4>), dim3(segs.nblocks), dim3(kBlock), 0, stream, lay, arp.p, aci.p, av.p, (const double *)x.p, d_b, tmp64a.p, partials.p, segs.ss); break;
     case 16: hipLaunchKernelGGL((k_spmv_res_seg<16>), dim3(segs.nblocks), dim3(kBlock), 0, stream, lay, arp.p, aci.p, av.p, (const double *)x.p, d_b, tmp64a.p, partials.p, segs.ss); break;
     case 32: hipLaunchKernelGGL((k_spmv_res_seg<32>), dim3(segs.nblocks), dim3(kBlock), 0, stream, lay, arp.p, aci.p, av.p, (const double *)x.p, d_b, tmp64a.p, partials.p, segs.ss); break;

@@ -68,6 +68,10 @@ struct RowMeta {
 // merged: the row may also hold right-hand sides of its own level group
 // (column c stored as -2 - c; see merge_plan.hpp), gathered from rhs.
 //
+// The matrix is loaded plainly at every size (both sweeps, non-temporal ->
+// plain: 97x61x83 FP32 0.33 -> 0.31 ms, 128^3 FP32 0.73 -> 0.70 ms, 256^3 2.60
+// -> 2.55 ms: it comes back from the Infinity Cache as far as it fits it).
+//
 // px >= 0: the row whose value the last round waits for before it gathers (a
 // proxy of its latest dependencies, see row_proxy).  A wave is usually at
 // its task long before its inputs are: gathering them then, and again once
@@ -294,8 +298,9 @@ __global__ __launch_bounds__(256) void k_sptrsv(
     const int *__restrict__ wave_ptr, const SweepTask *__restrict__ wt,
     const int *__restrict__ slot_row, const int *__restrict__ rp, const int *__restrict__ ci,
     const VT *__restrict__ cv, const int *__restrict__ mrp, const int *__restrict__ mci,
-    const VT *__restrict__ mcv, const VT *__restrict__ diag, const BT *__restrict__ rhs, XT *x, XT *__restrict__ aux, const double *__restrict__ dotv,
-    double *__restrict__ partials, DevScalars *sc, const int *stop, int defer, int coherent) {
+    const VT *__restrict__ mcv, const VT *__restrict__ diag, const BT *__restrict__ rhs, XT *x,
+    XT *__restrict__ aux, const double *__restrict__ dotv, double *__restrict__ partials,
+    DevScalars *sc, const int *stop, int defer, int coherent) {
   if (*stop) return;
   const int lane = threadIdx.x & 63;
   const int wave =  // wave-uniform: the list comes through the scalar cache

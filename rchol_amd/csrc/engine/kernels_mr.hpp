@@ -1,9 +1,9 @@
 // Multi-right-hand-side kernels: K columns stored interleaved (row-major
 // n x K, element (i, c) at i*K + c).  A lane owns one column (sweeps) or kCols
-// neighbouring ones, so K or K / kCols lanes apply a matrix entry (index + value, loaded once) to K
-// columns with one coalesced K-wide vector access.  Every
-// column runs its own PCG recurrence (pcg.cpp:57-127) with its own scalars
-// and convergence mask; a converged column is frozen.
+// neighbouring ones, so K or K / kCols lanes apply a matrix entry (index +
+// value, loaded once) to K columns with one coalesced K-wide vector access.
+// Every column runs its own PCG recurrence (pcg.cpp:57-127) with its own
+// scalars and convergence mask; a converged column is frozen.
 #pragma once
 #include "kernels.hpp"
 
@@ -290,7 +290,8 @@ __global__ __launch_bounds__(256) void k_sptrsv_mr(
     if (k + 1 < k1) fetch(k + 1);
 #define RCHOL_MR_TASK(LE)                                                                  \
   sweep_task_mr<VT, XT, BT, K, ((LE) * K <= 64 ? (LE) : 64 / K), FUSE>(                    \
-      cnt, m_row, m_e0, m_e1, m_dg, merged ? mci : ci, merged ? mcv : cv, rhs, x, aux, dotv, err, dacc[0][0], merged)
+      cnt, m_row, m_e0, m_e1, m_dg, merged ? mci : ci, merged ? mcv : cv, rhs, x, aux, dotv, \
+      err, dacc[0][0], merged)
     switch (lg) {
       case 0: RCHOL_MR_TASK(1); break;
       case 1: RCHOL_MR_TASK(2); break;
@@ -413,18 +414,15 @@ __global__ __launch_bounds__(256) void k_p_update_mr(int n, const ZT *__restrict
 }
 
 // q = A p, per-column p.r and p.q -> alpha_c.  Bound by the K-wide gathers of p
-// from the XCDs' L2 and the Infinity Cache:
-// 100^3, K = 32, FP32 factor: p update and SpMV 405 us, 1408 us before, when one
-// lane per column gathered z and p_old for every entry and one thread per column
-// walked the blocks' partials.
+// that leave the XCDs' L2 (256^3, K = 32: 35.1 GB in 6.0 ms, 5.8 TB/s, for 14.4 GB
+// of arrays).  100^3, K = 32, FP32 factor: p update and SpMV 405 us, 1408 us
+// before, when one lane per column gathered z and p_old for every entry and one
+// thread per column walked the blocks' partials.
 template <int K>
-__global__ __launch_bounds__(256, kSpmvMrBlocksPerCu) void k_spmv_p_mr(int n, const int *__restrict__ rp,
-                                                   const int *__restrict__ ci,
-                                                   const double *__restrict__ av,
-                                                   const double *__restrict__ p,
-                                                   double *__restrict__ q,
-                                                   const double *__restrict__ r,
-                                                   double *partials, BatchScalars *bs) {
+__global__ __launch_bounds__(256, kSpmvMrBlocksPerCu) void k_spmv_p_mr(
+    int n, const int *__restrict__ rp, const int *__restrict__ ci, const double *__restrict__ av,
+    const double *__restrict__ p, double *__restrict__ q, const double *__restrict__ r,
+    double *partials, BatchScalars *bs) {
   if (bs->all_done) return;
   const int col = threadIdx.x % (K / kCols) * kCols;
   const RowWalk rw = xcd_rows_mr<K>(n);
@@ -504,13 +502,10 @@ __global__ __launch_bounds__(256) void k_update_mr(int n, const double *__restri
 // Per-column true residual ||A x - b|| / ||b|| (pcg.cpp:116-118); with
 // bvec == null a plain Y = A X.
 template <int K>
-__global__ __launch_bounds__(256, kSpmvMrBlocksPerCu) void k_spmv_res_mr(int n, const int *__restrict__ rp,
-                                                     const int *__restrict__ ci,
-                                                     const double *__restrict__ av,
-                                                     const double *__restrict__ x,
-                                                     const double *__restrict__ bvec,
-                                                     double *__restrict__ y, double *partials,
-                                                     BatchScalars *bs) {
+__global__ __launch_bounds__(256, kSpmvMrBlocksPerCu) void k_spmv_res_mr(
+    int n, const int *__restrict__ rp, const int *__restrict__ ci, const double *__restrict__ av,
+    const double *__restrict__ x, const double *__restrict__ bvec, double *__restrict__ y,
+    double *partials, BatchScalars *bs) {
   const int col = threadIdx.x % (K / kCols) * kCols;
   const RowWalk rw = xcd_rows_mr<K>(n);
   double aqq[1][kCols] = {{0.0, 0.0}};

@@ -51,9 +51,11 @@ constexpr int kMergeMaxLevels = 1 << 20;  // (fits the sort key of a merged entr
 // groups, to rows that grow at most kDeepGrowth-fold on average (24^3 in
 // natural order, 2929 levels, FP64: 48-fold 7.5 ms per solve and 40 ms of
 // planning, 96-fold 5.7 and 55; static 64^3, 8216 levels: 54 and 51 ms).
-// Planning grows with the levels and stays out beyond kDeepMaxLevels (static
-// 72^3, 10817 levels: 0.24 s; 256^3, 104163 levels: 4.5 s, for sweeps that the
-// chunks win).
+// Planning grows with the levels and stays out beyond kDeepMaxLevels.  That
+// line bounds the upload, not the gain: at static 96^3 (17126 levels) and 128^3
+// (21937) planning would take 0.46 and 0.68 s, the chunks' 0.11 and 0.22, for
+// sweeps of 5.6 and 9.9 ms an application instead of 9.0 and 15.1; at 256^3
+// (104163) 4.5 s, for sweeps that the chunks win.
 #ifndef RCHOL_AMD_MERGE_DEEP_CAP
 #define RCHOL_AMD_MERGE_DEEP_CAP 0.05
 #endif

@@ -1846,22 +1846,28 @@ int setup_chunks(rchol_amd_ctx *c, size_t n, HostSweep &hf, HostSweep &hb, int n
 }
 
 // Whether the merged levels of a deep factor take the place of its chunks: by
-// the estimates, the chunks' raised by half where chunks read each other (the
-// hand-over from chunk to chunk takes longer than estimated).
+// the estimates, weighed by what they were measured to be worth.  The hand-over
+// from chunk to chunk takes longer than estimated, so chunks that read each
+// other count for more than chunks that do not (stacks of small systems).
 //
-// Both forms of 41 factors (natural and static orders of 2D and 3D grids from
-// 64^2 to 1000x600 and 14^3 to 88^3, chains, and stacks of 4 to 2000 of them;
-// FP64 / FP32, merged over chunked time of one application) against merged
-// over chunked estimate:
-//   chunks that read each other: 0.15 ... 0.56 at estimates 0.1 ... 0.55 (0.74
-//   at most), 0.62 / 0.67 at 1.01 (static 72^3), 0.60 / 0.63 at 1.24 (88^3),
-//   0.72 / 0.76 at 1.41 (160x160x20); 1.56 / 1.67 at 1.96, 1.87 / 1.76 at 2.78
-//   (stacks of 32 natural 16^3 and 16 static 32^3)
-//   chunks that do not: 0.61 / 0.71 at 0.93 (256 chains of 2000 rows), 1.24 /
-//   1.50 at 1.01 (32 natural 64x64 grids), 2.24 / 2.58 at 2.69 (128 of them)
+// One application of 70 factors (natural and static orders of 2D and 3D grids
+// from 64^2 to 1000x600 and 14^3 to 88^3, chains, and stacks of 2 to 2000 of
+// them), merged over chunked time (FP64 / FP32), by the estimates' ratio:
+//   chunks that read each other: merged wins below a ratio of 1 (0.87 / 0.84 at
+//   0.86, 4 static 32^3, at most), 0.62 / 0.67 at 1.01 (static 72^3), 0.60 /
+//   0.63 at 1.24 (88^3), 0.72 / 0.76 at 1.41 (160x160x20); 1.30 / 1.23 at 1.47
+//   and 1.87 / 1.76 at 2.78 (8 and 16 static 32^3)
+//   chunks that do not: 0.60 / 0.71 at 0.93 (256 chains of 2000 rows), 1.04 /
+//   1.16 at 0.83 (8 natural 26^3); 1.05 / 1.35 at 0.96 (16 natural 16^3), 1.11 /
+//   1.31 at 0.98, 1.45 / 1.72 at 1.13 and 1.95 / 2.20 at 1.53 (32, 40 and 64
+//   natural 64x64); chains by the hundred are the exception, 0.39 / 0.48 at 1.32
+//   (400 of them: the time of many chunks grows with their number, which the
+//   estimate leaves out)
+constexpr double kLinkedWeight = 1.45, kUnlinkedWeight = 0.95;
 bool merged_wins(const rchol_amd_ctx *c, const MergePlan &f, const MergePlan &b) {
   return f.any() && b.any() &&
-         f.est_us + b.est_us < (c->chunks_linked ? 1.5 : 1.0) * c->chunk_est_us;
+         f.est_us + b.est_us <
+             (c->chunks_linked ? kLinkedWeight : kUnlinkedWeight) * c->chunk_est_us;
 }
 
 }  // namespace

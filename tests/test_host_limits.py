@@ -100,6 +100,8 @@ def test_plans_without_all_their_threads(system, tmp_path, threads):
     out = str(tmp_path / "out.npz")
     p = child(system, out, big_stacks)
     print(p.stdout)
+    if "threads" not in p.stdout:
+        pytest.skip("the interpreter itself does not fit the limit")
     if "threads 8" in p.stdout:
         pytest.skip("every thread could be started")
     assert p.returncode == 0, (p.returncode, p.stdout, p.stderr)
